@@ -281,7 +281,9 @@ __global__ __launch_bounds__(64 * S) void skinny_row_kernel(const int8_t* __rest
   constexpr int kPast = 0x7FFFFFF0;
   const v4u q8_buf = wide_buffer(q8, (long long)m * q8_stride);
   const v4u w_buf = wide_buffer(packed, (long long)a.rows * a.row_bytes);
-  const v4u s_buf = wide_buffer(scales, (long long)a.rows * a.groups * 2);
+  // The scales are fetched as dwords and the range check drops a dword that ends past the size: an odd
+  // count of halfwords is rounded up, so that the last scale's dword counts (it shares its dword's page).
+  const v4u s_buf = wide_buffer(scales, ((long long)a.rows * a.groups * 2 + 3) & ~3LL);
 
   // What the epilogue reads from global memory (token scales, biases, residual
   // bases of this thread's outputs) goes out first: older than every
