@@ -408,10 +408,6 @@ __device__ __forceinline__ v4f32 load_f128(const void* p) {
   asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(r) : "v"(p) : "memory");
   return r;
 }
-// A value u = fma(x, 1/s, 128) at least this far below the next half-integer
-// and above the previous one rounds like x/s + 128 (see quantize_row_split).
-constexpr float kTieGuard = 0.49997f;
-
 // f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): an
 // unrolled loop whose index can feed an immediate operand.
 template <int N, int I = 0, typename F>
@@ -433,15 +429,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 // caller issues weight loads there).  slots holds T/64 floats.  The LDS
 // writes are not yet waited for.
 //
-// Bit-exact with the quantizer kernels (quantize_plain_slice):
-// scale = max(amax/127, 1e-5) and q = (int)rint(x / scale).  The division is
-// replaced by u = RN(x * inv + 128) with inv = RN(1/scale), q + 128 = rint(u):
-// |x/scale| <= 127 * (1 + 2^-23), so |x*inv - x/scale| <= 127 * 2^-24 and the
-// fma's rounding adds at most 2^-17 (half an ulp below 256), |u - (x/scale + 128)|
-// < 1.6e-5; the correctly rounded quotient is within 2^-18 of x/scale.  When u
-// lies more than 2e-5 from every half-integer, rint(u) - 128 is therefore
-// rint(RN(x/scale)).  Closer values (about 6 in 10^5 inputs, exact ties among
-// them), NaN and infinities take the division itself.
+// Bit-exact with the quantizer kernels (quantize4).
 //
 // Layout: the lanes 4g .. 4g + 3 hold the four float4 of one 16-input quad g;
 // q8 word k of the quad holds inputs 4b + k at byte b, so lane j (= t & 3)
@@ -480,14 +468,9 @@ __device__ __forceinline__ float quantize_row_split(v4f32 (&xv)[X], int n, int c
   for (int w = 1; w < T / 64; ++w) amax = fmaxf(amax, slots[w]);
   const float scale = fmaxf(amax / 127.0f, 1e-5f);
   const float inv = 1.0f / scale;
-  // Per-lane constants: v_perm_b32 selectors (byte values 0..3 pick from the
-  // second operand, 4..7 from the first, 0x0C gives zero) and the split's
-  // rotation and nibble mask.
-  unsigned sel_near = 0x0C0C0C0Cu, sel_far = 0x0C0C0C0Cu;
-  sel_near = (sel_near & ~(0xFFu << (8 * j))) | ((unsigned)j << (8 * j));                  // own byte j at j
-  sel_near = (sel_near & ~(0xFFu << (8 * (j ^ 1)))) | ((unsigned)(4 + j) << (8 * (j ^ 1)));  // lane j^1's at j^1
-  sel_far = (sel_far & ~(0xFFu << (8 * (j ^ 2)))) | ((unsigned)j << (8 * (j ^ 2)));          // lane j^2's at j^2
-  sel_far = (sel_far & ~(0xFFu << (8 * (j ^ 3)))) | ((unsigned)(4 + j) << (8 * (j ^ 3)));    // lane j^3's at j^3
+  // Per-lane constants: the transpose's selectors and the split's rotation and
+  // nibble mask.
+  const QuadTranspose transpose(j);
   const unsigned rot = j < 2 ? 4u : 28u;
   const unsigned nibbles = j < 2 ? 0x0F0F0F0Fu : 0xF0F0F0F0u;
   // float4 f = k*T + tid is quad g = f >> 2 (chunk g >> 2, quad g & 3) and
@@ -497,28 +480,9 @@ __device__ __forceinline__ float quantize_row_split(v4f32 (&xv)[X], int n, int c
   static_for<X>([&](auto kc) {
     constexpr int k = decltype(kc)::value;
     const int f = k * T + tid;
-    float v[4];
-    bool near = false;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float u = __builtin_fmaf(xv[k][e], inv, 128.0f);
-      const float r = __builtin_rintf(u);
-      near = near || !(fabsf(u - r) < kTieGuard);
-      v[e] = r;
-    }
-    if (near) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = (float)((int)__builtin_rintf(xv[k][e] / scale) + 128);
-    }
-    unsigned biased = __builtin_amdgcn_cvt_pk_u8_f32(v[0], 0, 0u);
-    biased = __builtin_amdgcn_cvt_pk_u8_f32(v[1], 1, biased);
-    biased = __builtin_amdgcn_cvt_pk_u8_f32(v[2], 2, biased);
-    biased = __builtin_amdgcn_cvt_pk_u8_f32(v[3], 3, biased);
-    const unsigned q4 = biased ^ 0x80808080u;  // the four q bytes
-    const unsigned p1 = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0xB1, 0xF, 0xF, false);  // lane ^ 1
-    const unsigned p2 = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x4E, 0xF, 0xF, false);  // lane ^ 2
-    const unsigned p3 = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x1B, 0xF, 0xF, false);  // lane ^ 3
-    const unsigned word = __builtin_amdgcn_perm(p1, q4, sel_near) | __builtin_amdgcn_perm(p3, p2, sel_far);
+    const float e[4] = {xv[k][0], xv[k][1], xv[k][2], xv[k][3]};
+    const unsigned q4 = quantize4(e, inv, scale);  // the four q bytes
+    const unsigned word = transpose.word(q4);
     const unsigned partner = (unsigned)__builtin_amdgcn_mov_dpp((int)word, 0x4E, 0xF, 0xF, false);  // lane ^ 2
     const unsigned turned = __builtin_amdgcn_alignbit(word, word, rot);
     const unsigned split = (turned & nibbles) | (partner & ~nibbles);

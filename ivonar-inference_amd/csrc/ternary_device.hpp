@@ -263,13 +263,18 @@ constexpr int kBatch = 16;
 // lanes 0 and 32 only: at stage o every lane their sums depend on is below o
 // within its half, so L ^ o = L + o, the lane a DPP row shift (o < 16) or
 // the row swap (o = 16) reads; same operands, same order.
-__device__ __forceinline__ float tree_reduce(float s, float* slots) {
-  const int tid = threadIdx.x;
+__device__ __forceinline__ float half_wave_sum(float s) {
   s = s + row_swap16(s);
   s = s + row_shl<8>(s);
   s = s + row_shl<4>(s);
   s = s + row_shl<2>(s);
   s = s + row_shl<1>(s);
+  return s;
+}
+
+__device__ __forceinline__ float tree_reduce(float s, float* slots) {
+  const int tid = threadIdx.x;
+  s = half_wave_sum(s);
   if ((tid & 31) == 0) slots[tid >> 5] = s;
   __syncthreads();
   float total = 0.0f;
@@ -315,6 +320,62 @@ __device__ __forceinline__ float source_value(const float* __restrict__ input, i
     return input[i];
   }
 }
+
+// A value u = fma(x, 1/s, 128) at least this far below the next half-integer
+// and above the previous one rounds like x/s + 128 (see quantize4).
+constexpr float kTieGuard = 0.49997f;
+
+// The int8 values (int)rint(x[e] / scale) of four inputs, input e at byte e,
+// for |x| <= 127 * scale (1 + 2^-23) with scale = max(amax/127, 1e-5) and
+// inv = RN(1/scale).  The division is replaced by u = RN(x * inv + 128),
+// q + 128 = rint(u): |x*inv - x/scale| <= 127 * 2^-24 and the fma's rounding
+// adds at most 2^-17 (half an ulp below 256), |u - (x/scale + 128)| < 1.6e-5;
+// the correctly rounded quotient is within 2^-18 of x/scale.  When u lies more
+// than 2e-5 from every half-integer, rint(u) - 128 is therefore
+// rint(RN(x/scale)).  Closer values (about 6 in 10^5 inputs, exact ties among
+// them), NaN and infinities take the division itself.
+__device__ __forceinline__ unsigned quantize4(const float (&x)[4], float inv, float scale) {
+  float v[4];
+  bool near = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float u = __builtin_fmaf(x[e], inv, 128.0f);
+    const float r = __builtin_rintf(u);
+    near = near || !(fabsf(u - r) < kTieGuard);
+    v[e] = r;
+  }
+  if (near) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (float)((int)__builtin_rintf(x[e] / scale) + 128);
+  }
+  unsigned biased = __builtin_amdgcn_cvt_pk_u8_f32(v[0], 0, 0u);
+  biased = __builtin_amdgcn_cvt_pk_u8_f32(v[1], 1, biased);
+  biased = __builtin_amdgcn_cvt_pk_u8_f32(v[2], 2, biased);
+  biased = __builtin_amdgcn_cvt_pk_u8_f32(v[3], 3, biased);
+  return biased ^ 0x80808080u;
+}
+
+// The q8 words of a 16-input quad from its four lanes' bytes (lanes 4g .. 4g+3,
+// lane j holds inputs 4j .. 4j+3): word k of the quad takes byte k of lane i
+// at byte i, so lane j forms word j with three DPP quad permutations and two
+// v_perm_b32 (byte values 0..3 pick from the second operand, 4..7 from the
+// first, 0x0C gives zero).
+struct QuadTranspose {
+  unsigned near, far;
+  __device__ __forceinline__ explicit QuadTranspose(int j) {
+    near = far = 0x0C0C0C0Cu;
+    near = (near & ~(0xFFu << (8 * j))) | ((unsigned)j << (8 * j));                    // own byte j at j
+    near = (near & ~(0xFFu << (8 * (j ^ 1)))) | ((unsigned)(4 + j) << (8 * (j ^ 1)));  // lane j^1's at j^1
+    far = (far & ~(0xFFu << (8 * (j ^ 2)))) | ((unsigned)j << (8 * (j ^ 2)));          // lane j^2's at j^2
+    far = (far & ~(0xFFu << (8 * (j ^ 3)))) | ((unsigned)(4 + j) << (8 * (j ^ 3)));    // lane j^3's at j^3
+  }
+  __device__ __forceinline__ unsigned word(unsigned q4) const {
+    const unsigned p1 = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0xB1, 0xF, 0xF, false);  // lane ^ 1
+    const unsigned p2 = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x4E, 0xF, 0xF, false);  // lane ^ 2
+    const unsigned p3 = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x1B, 0xF, 0xF, false);  // lane ^ 3
+    return __builtin_amdgcn_perm(p1, q4, near) | __builtin_amdgcn_perm(p3, p2, far);
+  }
+};
 
 // Everything a block needs to quantize one token row.
 struct RowSource {
@@ -422,7 +483,7 @@ template <int MODE, int NB = kBatch, typename AfterLoads = NoLoads>
 __device__ __forceinline__ float quantize_row_to_lds(const RowSource& src, int chunks, unsigned char* lds_q,
                                                      float* slots, AfterLoads after_loads = AfterLoads{}) {
   static_assert(MODE == kPlain || MODE == kNorm, "register path for PLAIN and NORM rows");
-  static_assert(NB >= 1 && NB <= kBatch, "at most kBatch inputs per thread");
+  static_assert(NB >= 1 && NB <= 2 * kBatch, "at most 32 inputs per thread");
   const int tid = threadIdx.x;
   const int n = src.n;
   float v[NB], w[NB];
@@ -456,6 +517,7 @@ __device__ __forceinline__ float quantize_row_to_lds(const RowSource& src, int c
   amax = block_max(amax, slots + 32);
   const float scale = fmaxf(amax / 127.0f, 1e-5f);
   if constexpr (NB % 4 == 0) {
+    const float inv = 1.0f / scale;
     // Thread t's input t + 256b is byte j = (t >> 2) & 3 of word (chunk
     // (t >> 6) + 4b, quad (t >> 4) & 3, field t & 3): the four bytes of a word
     // sit in lanes 4 apart within a 16-lane row, one per j.  For each four
@@ -475,13 +537,10 @@ __device__ __forceinline__ float quantize_row_to_lds(const RowSource& src, int c
     const unsigned sel_b = place(place(0x0C0C0C0Cu, jb, (unsigned)j), jc, 4u + j);  // lanes jb and jc
 #pragma unroll
     for (int c = 0; c < NB / 4; ++c) {
-      unsigned q4 = 0;
+      float e4[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int i = (4 * c + e) * kThreads + tid;
-        const int q = i < n ? (int)__builtin_rintf(v[4 * c + e] / scale) : 0;
-        q4 |= ((unsigned)q & 0xffu) << (8 * e);
-      }
+      for (int e = 0; e < 4; ++e) e4[e] = (4 * c + e) * kThreads + tid < n ? v[4 * c + e] : 0.0f;
+      const unsigned q4 = quantize4(e4, inv, scale);
       const unsigned pa = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x124, 0xF, 0xF, false);
       const unsigned pb = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x128, 0xF, 0xF, false);
       const unsigned pc = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x12C, 0xF, 0xF, false);
@@ -531,94 +590,21 @@ __device__ __forceinline__ float quantize_plain_row4_to_lds(const RowSource& src
   }
   amax = block_max(amax, slots + 32);
   const float scale = fmaxf(amax / 127.0f, 1e-5f);
-  // The four lanes 4g .. 4g + 3 hold the four float4 of one 16-input quad;
-  // word k of the quad takes byte j of lane j's quantized float4 at byte j
-  // (inputs 16w + k + 4j), so lane j forms word j with three DPP quad
-  // permutations and two v_perm_b32 (the byte transpose of
-  // quantize_row_split) and stores it whole.
+  const float inv = 1.0f / scale;
   const int j = tid & 3;
-  unsigned sel_near = 0x0C0C0C0Cu, sel_far = 0x0C0C0C0Cu;
-  sel_near = (sel_near & ~(0xFFu << (8 * j))) | ((unsigned)j << (8 * j));
-  sel_near = (sel_near & ~(0xFFu << (8 * (j ^ 1)))) | ((unsigned)(4 + j) << (8 * (j ^ 1)));
-  sel_far = (sel_far & ~(0xFFu << (8 * (j ^ 2)))) | ((unsigned)j << (8 * (j ^ 2)));
-  sel_far = (sel_far & ~(0xFFu << (8 * (j ^ 3)))) | ((unsigned)(4 + j) << (8 * (j ^ 3)));
+  const QuadTranspose transpose(j);
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const int f = c * kThreads + tid;
     const float e[4] = {v[c].x, v[c].y, v[c].z, v[c].w};
-    unsigned q4 = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k)  // inputs past the row (f >= n4) hold zeros, which quantize to 0
-      q4 |= ((unsigned)(int)__builtin_rintf(e[k] / scale) & 0xffu) << (8 * k);
-    const unsigned p1 = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0xB1, 0xF, 0xF, false);  // lane ^ 1
-    const unsigned p2 = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x4E, 0xF, 0xF, false);  // lane ^ 2
-    const unsigned p3 = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x1B, 0xF, 0xF, false);  // lane ^ 3
-    const unsigned word = __builtin_amdgcn_perm(p1, q4, sel_near) | __builtin_amdgcn_perm(p3, p2, sel_far);
+    // Inputs past the row (f >= n4) hold zeros, which quantize to 0.
+    const unsigned word = transpose.word(quantize4(e, inv, scale));
     if (f < chunks * 16) {  // whole quads: chunks * 16 is a multiple of 4
       const int g = f >> 2;  // quad g: chunk g >> 2, quad g & 3
       reinterpret_cast<unsigned*>(lds_q)[(((g & 3) * chunks + (g >> 2)) << 2) + j] = word;
     }
   }
   return scale;
-}
-
-// One block's share of the PLAIN quantizer for a 16-byte aligned row of n
-// inputs (n a multiple of 4): T/16 chunks (slice `slice`), one q8 word per
-// thread.  Every thread issues all of its loads in one round - its four
-// inputs and its share of the row's amax as float4 (a row longer than
-// ROUNDS*T float4 takes more rounds) - so the slice costs one memory
-// round trip, a block max and the divisions.  Writes the slice's q8 words
-// (split_quad_word form if `split`), its chunk sums and, from slice 0, the
-// token scale.  slots holds T/64 floats; all threads of the block call it.
-template <int T, int ROUNDS = 8>
-__device__ __forceinline__ void quantize_plain_slice(const float* __restrict__ row, int n, int slice, bool split,
-                                                     int8_t* __restrict__ q8, int32_t* __restrict__ xsum,
-                                                     float* __restrict__ scale_out, float* slots) {
-  constexpr int kSlice = T / 16;  // chunks per block
-  const int tid = threadIdx.x;
-  const int n4 = n >> 2;
-  const int chunks = (n + kChunk - 1) / kChunk;
-  const float4* row4 = reinterpret_cast<const float4*>(row);
-
-  // This thread's q8 word: chunk u, quad w, field k holds inputs
-  // u*64 + w*16 + k + 4b for b = 0..3.
-  const int u = slice * kSlice + (tid >> 4);
-  const int first = u * kChunk + ((tid >> 2) & 3) * 16 + (tid & 3);
-  float mine[4];
-#pragma unroll
-  for (int b = 0; b < 4; ++b) mine[b] = row[min(first + 4 * b, n - 1)];
-  float amax = 0.0f;
-  for (int base = 0; base < n4; base += ROUNDS * T) {
-    float4 v[ROUNDS];
-#pragma unroll
-    for (int j = 0; j < ROUNDS; ++j) v[j] = row4[min(base + j * T + tid, n4 - 1)];
-#pragma unroll
-    for (int j = 0; j < ROUNDS; ++j)
-      amax = fmaxf(fmaxf(amax, fmaxf(fabsf(v[j].x), fabsf(v[j].y))), fmaxf(fabsf(v[j].z), fabsf(v[j].w)));
-  }
-  amax = wave_max(amax);
-  if ((tid & 63) == 0) slots[tid >> 6] = amax;
-  __syncthreads();
-  amax = slots[0];
-#pragma unroll
-  for (int w = 1; w < T / 64; ++w) amax = fmaxf(amax, slots[w]);
-  const float scale = fmaxf(amax / 127.0f, 1e-5f);
-
-  unsigned word = 0;
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    const int q = first + 4 * b < n ? (int)__builtin_rintf(mine[b] / scale) : 0;
-    word |= ((unsigned)q & 0xffu) << (8 * b);
-  }
-  const int value = (int)word;
-  const int total = chunk_lane_sum(word_sum(value));
-  const unsigned partner = (unsigned)__builtin_amdgcn_mov_dpp(value, 0x4E, 0xF, 0xF, false);  // lane ^ 2
-  if (u < chunks) {
-    int32_t* q8w = reinterpret_cast<int32_t*>(q8);
-    q8w[u * 16 + (tid & 15)] = split ? (int)split_quad_word(word, partner, tid & 3) : value;
-    if ((tid & 15) == 0) xsum[u] = total;
-  }
-  if (slice == 0 && tid == 0) *scale_out = scale;
 }
 
 // Hand-over between the blocks of one launch (the argmax's per-block pairs,

@@ -1,0 +1,84 @@
+"""The quantizer's register-resident rows at the edges of their layouts, bit for bit against the oracle:
+each row length one past or at a kernel's capacity, odd lengths, rows that start off a 16-byte boundary, and
+lengths past the last layout (the slice kernel)."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import ternary_oracle as T
+from _util import assert_bits_equal, to_np
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(actual, expected):
+    for what, a, e in zip(("q8", "xsum", "scale"), actual, expected):
+        assert_bits_equal(to_np(a), e, what)
+
+
+def _rows(rng, m, n):
+    x = (rng.standard_normal((m, n)) * rng.choice([1e-4, 1.0, 30.0], size=(m, 1))).astype(np.float32)
+    x[0] = np.rint(x[0] * 4) / 2  # ties at half-integer quotients where the scale allows them
+    x[0, n // 2] = 63.5
+    return x
+
+
+@pytest.mark.parametrize("m,n", [(3, 1028), (2, 4100), (513, 2052), (512, 4100), (513, 8192), (2, 8196), (2, 16388),
+                                 (1, 32768), (1, 32772), (2, 1023), (3, 2049), (2, 4097), (1, 8191), (1, 8193)])
+def test_plain_rows(cuda, oracle, m, n):
+    import torch
+    from ivonar_amd import ops
+
+    x = _rows(np.random.default_rng(m + n), m, n)
+    _check(ops.quantize_rows(torch.from_numpy(x).to(cuda)), oracle.quantize_rows(T.MODE_PLAIN, x, n))
+
+
+@pytest.mark.parametrize("n,stride,offset", [(1024, 1027, 1), (4096, 4098, 2), (8192, 8193, 3), (6000, 6004, 4)])
+def test_plain_rows_off_alignment(cuda, oracle, n, stride, offset):
+    import torch
+    from ivonar_amd import ops
+
+    x = _rows(np.random.default_rng(n), 3, n)
+    flat = torch.full((3 * stride + 8,), 7.0, device=cuda)
+    rows = flat[offset:offset + 3 * stride].view(3, stride)[:, :n]
+    rows.copy_(torch.from_numpy(x))
+    _check(ops.quantize_rows(rows, n=n), oracle.quantize_rows(T.MODE_PLAIN, x, n))
+
+
+@pytest.mark.parametrize("n", [1, 1025, 2048, 2049, 4097, 8191, 8193])
+def test_norm_rows(cuda, oracle, n):
+    import torch
+    from ivonar_amd import ops
+
+    rng = np.random.default_rng(n)
+    x = _rows(rng, 3, n)
+    weight = (1.0 + 0.1 * rng.standard_normal(n)).astype(np.float32)
+    actual = ops.quantize_rows(torch.from_numpy(x).to(cuda), mode=ops.MODE_NORM, aux=torch.from_numpy(weight).to(cuda))
+    _check(actual, oracle.quantize_rows(T.MODE_NORM, x, n, aux=weight, eps=1e-6))
+
+
+# head_dim * heads inputs: one, two, four and eight words per thread, pairs beyond the LDS table (5000), and
+# rows beyond the last layout.
+@pytest.mark.parametrize("head_dim,heads,splits", [(64, 64, 1), (64, 65, 8), (48, 171, 3), (128, 128, 2),
+                                                   (64, 512, 8), (5, 1000, 5), (64, 513, 1)])
+def test_attn_rows(cuda, oracle, head_dim, heads, splits):
+    import torch
+    from ivonar_amd import ops, runtime
+
+    rng = np.random.default_rng(head_dim + heads)
+    parts = rng.standard_normal((2, heads, splits, head_dim + 2)).astype(np.float32)
+    parts[..., 0] *= 8.0
+    parts[..., 1] = np.abs(parts[..., 1]) + 0.5
+    if splits > 1:
+        parts[0, 3, 1, 0] = -np.inf  # an empty split
+    n, stride = heads * head_dim, heads * splits * (head_dim + 2)
+    flat = parts.reshape(2, stride)
+    assert runtime.library().ivonar_define(b"HEAD_DIM", head_dim) == 0
+    try:
+        actual = ops.quantize_rows(torch.from_numpy(flat).to(cuda), mode=ops.MODE_ATTN, splits=splits, n=n)
+        _check(actual, oracle.quantize_rows(T.MODE_ATTN, flat, n, splits=splits, head_dim=head_dim, m=2,
+                                            in_stride=stride))
+    finally:
+        runtime.library().ivonar_define(b"HEAD_DIM", 64)
