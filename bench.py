@@ -799,7 +799,7 @@ def main() -> None:
 
 
 def decode_stack(device, generated: int = 256, repeats: int = 3, sampling=None):
-    """Decode on the 24-layer d=1024 stack (vocab 32000, 36-token prompt): prefill in 32-token tiles,
+    """Decode on the 24-layer d=1024 stack (vocab 32000, 36-token prompt): prefill in one 64-token tile,
     then `generated` tokens in 16-step HIP-graph bursts with one token read-back per burst.  Greedy, or
     with `sampling` = (temperature, top_k, repetition penalty) drawn by the device sampler.  tok/s counts
     the decode steps only; the wall clock includes the read-backs."""
@@ -851,8 +851,8 @@ def decode_stack(device, generated: int = 256, repeats: int = 3, sampling=None):
         "ms_per_token": round(best / generated * 1e3, 4),
         "prefill_36_ms": round(min(prefill_times) * 1e3, 3),
         "prefill_36_ms_eager": round(min(eager_prefill) * 1e3, 3),
-        "prefill_note": "two 32-token tiles and the head; prefill_36_ms replays the captured tile graph once per "
-                        "tile, prefill_36_ms_eager launches the same program call by call",
+        "prefill_note": "one 64-token tile and the head; prefill_36_ms replays the captured graph of that tile "
+                        "size, prefill_36_ms_eager launches the same program call by call",
         "weight_bytes_per_token": decoder_bytes(config),
         "tokens_first8": tokens[:8],
         "tokens_sha1": hashlib.sha1(",".join(map(str, tokens)).encode()).hexdigest()[:16],

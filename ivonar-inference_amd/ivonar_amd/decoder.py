@@ -18,12 +18,14 @@ decode step (``kernel_decoder.py:233-269``)::
     ivonar_argmax                                 logits -> next token (greedy)
       or, with sampling: uniform_(), logit_bounds, sample_token (kernel_decoder.py:619-681)
 
-prefill tile (``kernel_decoder.py:303-368``): ``embed_tile``, per layer
-``quantize_tile_norm`` + ``gemm_tile_store``, ``quantize_tile_plain`` +
-``gemm_tile_residual``, ``quantize_tile_norm`` + ``gemm_tile_silu_pair``,
-``quantize_tile_plain`` + ``gemm_tile_residual``, then ``gather_token``; the
-head and the first token's selection run once, after the last tile (the
-reference runs its head in every tile and samples after the prompt).
+prefill tile (``kernel_decoder.py:303-368``): ``embed_tile``, per layer a NORM
+quantization + ``gemm_tile_store``, PLAIN + ``gemm_tile_residual``, NORM +
+``gemm_tile_silu_pair``, PLAIN + ``gemm_tile_residual``, then ``gather_token``;
+the head and the first token's selection run once, after the last tile (the
+reference runs its head in every tile and samples after the prompt).  The
+reference's tile has 32 tokens; here a tile is the smallest of ``TILES`` that
+holds what is left of the prompt, since a tile's 194 dependent launches (24
+layers) cost the same 3 to 4 us each at 32 tokens as at 256.
 
 The mixers (recurrent scan, latent attention) are not part of this path: the
 output projection reads the V third of the entry projection's output instead
@@ -43,11 +45,17 @@ import torch
 from . import runtime
 from .matrix import Matrix, _lanes_for
 from .quantization import TernaryLinear
+from .ops import MODE_NORM, MODE_PLAIN
 from .runtime import KernelError, Launch, float32, int32, pointer
 from .sampling import DeviceSampler
 from .synthetic import LinearStackWeights
 
 TILE = 32
+# Tokens per prefill tile, each a launch list of its own (and a graph, after capture()).  Up to 1024 tokens
+# a tile costs less than two of half its size, padding included (24 layers of 1024/4096, graph replays of 32,
+# 64, .. 1024 tokens: 657, 722, 849, 1136, 1457, 2178 us; sizes between them, 192, 384 and 768, saved under 5%).
+# A prompt of 500 tokens took 11.25 ms in 16 tiles of 32 and takes 1.54 ms in one of 512.
+TILES = (32, 64, 128, 256, 512, 1024)
 SELF_CHECK_TOLERANCE = 0.25  # kernel_decoder.py:38
 THREADS = 256
 HEAD_LANES = 4
@@ -122,24 +130,28 @@ class StackDecoder:
         self.sampler = DeviceSampler(vocab, device, max_top_k) if sampling else None
         self.uniforms = torch.zeros(self.burst, **f32)
         self.drawn_uniforms: list[float] = []  # with sampling: the uniform of every token advance_many returned
-        # prefill tile buffers (kernel_decoder.py:308-319)
-        self.tile_tokens = torch.zeros(TILE, dtype=torch.int64, device=device)
-        self.tile_valid = torch.zeros(1, dtype=torch.int64, device=device)
-        self.residual_tile = torch.zeros(TILE, hidden, **f32)
-        self.mixer_in_tile = torch.zeros(TILE, config.qkv, **f32)
-        self.ffn_tile = torch.zeros(TILE, dense, **f32)
-        self.q8_tile = torch.zeros(TILE, max_chunks * CHUNK, dtype=torch.int8, device=device)
-        self.xsum_tile = torch.zeros(TILE, max_chunks, dtype=torch.int32, device=device)
-        self.scale_tile = torch.zeros(TILE, **f32)
+        # prefill tile buffers (kernel_decoder.py:308-319), for the longest tile: the count of valid tokens and
+        # their ids in one buffer, filled by one copy per tile
+        longest = TILES[-1]
+        self._tile_host = torch.zeros(1 + longest, dtype=torch.int64)
+        self.tile_input = torch.zeros(1 + longest, dtype=torch.int64, device=device)
+        self.tile_valid, self.tile_tokens = self.tile_input[:1], self.tile_input[1:]
+        self.residual_tile = torch.zeros(longest, hidden, **f32)
+        self.mixer_in_tile = torch.zeros(longest, config.qkv, **f32)
+        self.ffn_tile = torch.zeros(longest, dense, **f32)
+        self.q8_tile = torch.zeros(longest, max_chunks * CHUNK, dtype=torch.int8, device=device)
+        self.xsum_tile = torch.zeros(longest, max_chunks, dtype=torch.int32, device=device)
+        self.scale_tile = torch.zeros(longest, **f32)
         # The head is one GEMV with the RMSNorm prologue fused (the reference runs quantize_norm and
         # gemv_prequant_store, kernel_decoder.py:265-267; the logits are the same bits either way).
         self._head = [self._gemv("gemv_norm_store", self.token_matrix, self.residual, self.final_norm, self.logits,
                                  eps=config.eps)]
-        self._steps = [self._build_step(slot) for slot in range(self.burst)]
-        self._tile = self._build_tile()
+        layers = self._build_layers()
+        self._steps = [self._build_step(slot, layers) for slot in range(self.burst)]
+        self._tiles = self._build_tiles()
         self._first = self._head + self._select(self.burst - 1)  # after the last tile
         self._graph: torch.cuda.CUDAGraph | None = None
-        self._tile_graph: torch.cuda.CUDAGraph | None = None
+        self._tile_graph: dict[int, torch.cuda.CUDAGraph] | None = None  # one per tile size
         self.position = 0
 
     # ------------------------------------------------------------------ launch builders
@@ -167,23 +179,22 @@ class StackDecoder:
             name += "_wide"
         return Launch(self.module.kernel(name), (1, 1, 1), (THREADS, 1, 1), args)
 
-    def _quantize_tile(self, name: str, source, width: int, in_stride: int, aux=None, eps: float = 1e-6) -> Launch:
-        """kernel_decoder.py:370-386."""
-        args = [pointer(source), int32(in_stride), pointer(aux), int32(width), float32(eps), int32(1),
-                pointer(self.q8_tile), pointer(self.xsum_tile), pointer(self.scale_tile)]
-        if width > 4 * THREADS:
-            name += "_wide"
-        return Launch(self.module.kernel(name), (TILE, 1, 1), (THREADS, 1, 1), args)
+    def _quantize_tile(self, mode: int, source, width: int, in_stride: int, aux=None, eps: float = 1e-6):
+        """kernel_decoder.py:370-386, as a function of the token count."""
+        kernel = self.module.kernel("ivonar_quantize_rows")
+        head = [int32(mode), pointer(source), int32(in_stride), pointer(aux), int32(width), float32(eps), int32(1)]
+        tail = [pointer(self.q8_tile), pointer(self.xsum_tile), pointer(self.scale_tile)]
+        return lambda tokens: Launch(kernel, (tokens, 1, 1), (THREADS, 1, 1), [*head, int32(tokens), *tail])
 
-    def _gemm_tile(self, name: str, matrix: Matrix, output, out_stride: int) -> Launch:
-        """kernel_decoder.py:388-397."""
+    def _gemm_tile(self, name: str, matrix: Matrix, output, out_stride: int):
+        """kernel_decoder.py:388-397, as a function of the token count."""
+        kernel = self.module.kernel(name + "_wide" if matrix.wide else name)
         args = [pointer(self.q8_tile), pointer(self.xsum_tile), pointer(self.scale_tile),
                 pointer(matrix.packed), pointer(matrix.scales), pointer(matrix.bias), pointer(output),
                 int32(matrix.rows), int32(matrix.in_features), int32(matrix.row_bytes), int32(matrix.groups),
-                int32(matrix.lanes), int32(out_stride), int32(TILE)]
-        if matrix.wide:
-            name += "_wide"
-        return Launch(self.module.kernel(name), (matrix.grid, 1, 1), (THREADS, 1, 1), args)
+                int32(matrix.lanes), int32(out_stride)]
+        grid = (matrix.grid, 1, 1)
+        return lambda tokens: Launch(kernel, grid, (THREADS, 1, 1), [*args, int32(tokens)])
 
     def _select(self, slot: int) -> list:
         """The next token into ring slot `slot`: greedy argmax, or a draw of the device sampler with a
@@ -212,15 +223,11 @@ class StackDecoder:
             raise RuntimeError("this decoder was created without sampling")
         self.sampler.configure_sampling(temperature, top_k, repetition_penalty, penalized_ids)
 
-    def _build_step(self, slot: int) -> list[Launch]:
-        """One greedy decode step reading the token in slot-1 of the ring and writing slot."""
+    def _build_layers(self) -> list[Launch]:
+        """The layers of one decode step, shared by every ring slot's launch list."""
         config = self.config
         hidden = config.hidden
-        previous = self.history[(slot - 1) % self.burst:(slot - 1) % self.burst + 1]
-        token = self.token_matrix
-        launches = [Launch(self.module.kernel("embed_token"), ((hidden + THREADS - 1) // THREADS, 1, 1), (THREADS, 1, 1),
-                           [pointer(previous), pointer(token.packed), pointer(token.scales), pointer(self.residual),
-                            int32(hidden), int32(token.row_bytes), int32(token.groups)])]
+        launches = []
         values = self.mixer_in.narrow(0, 2 * hidden, hidden)
         for ops in self.layers:
             launches.append(self._gemv("gemv_norm_store", ops.entry, self.residual, ops.mixer_norm, self.mixer_in,
@@ -229,37 +236,43 @@ class StackDecoder:
             launches.append(self._gemv("gemv_norm_silu_pair", ops.gate_up, self.residual, ops.ffn_norm,
                                        self.ffn_mid, eps=config.eps))
             launches.append(self._gemv("gemv_plain_residual", ops.down, self.ffn_mid, None, self.residual))
-        launches.extend(self._head)
-        launches.extend(self._select(slot))
         return launches
 
-    def _build_tile(self) -> list[Launch]:
-        """One 32-token prefill tile, ending with its last valid token's residual in ``self.residual``."""
+    def _build_step(self, slot: int, layers: list[Launch]) -> list[Launch]:
+        """One greedy decode step reading the token in slot-1 of the ring and writing slot."""
+        hidden = self.config.hidden
+        previous = self.history[(slot - 1) % self.burst:(slot - 1) % self.burst + 1]
+        token = self.token_matrix
+        embed = Launch(self.module.kernel("embed_token"), ((hidden + THREADS - 1) // THREADS, 1, 1), (THREADS, 1, 1),
+                       [pointer(previous), pointer(token.packed), pointer(token.scales), pointer(self.residual),
+                        int32(hidden), int32(token.row_bytes), int32(token.groups)])
+        return [embed, *layers, *self._head, *self._select(slot)]
+
+    def _build_tiles(self) -> dict[int, list[Launch]]:
+        """Per tile size: one prefill tile of up to that many tokens, ending with its last valid token's
+        residual in ``self.residual``.  The sizes share every argument but the token count."""
         config = self.config
         hidden, dense, qkv = config.hidden, config.dense, config.qkv
         token = self.token_matrix
-        launches = [Launch(self.module.kernel("embed_tile"), ((hidden + THREADS - 1) // THREADS, TILE, 1),
-                           (THREADS, 1, 1),
-                           [pointer(self.tile_tokens), pointer(token.packed), pointer(token.scales),
-                            pointer(self.residual_tile), int32(hidden), int32(token.row_bytes), int32(token.groups),
-                            int32(TILE)])]
+        embed = [pointer(self.tile_tokens), pointer(token.packed), pointer(token.scales),
+                 pointer(self.residual_tile), int32(hidden), int32(token.row_bytes), int32(token.groups)]
+        blocks = (hidden + THREADS - 1) // THREADS
+        steps = [lambda tokens: Launch(self.module.kernel("embed_tile"), (blocks, tokens, 1), (THREADS, 1, 1),
+                                       [*embed, int32(tokens)])]
         values = self.mixer_in_tile.narrow(1, 2 * hidden, hidden)
         for ops in self.layers:
-            launches.append(self._quantize_tile("quantize_tile_norm", self.residual_tile, hidden, hidden,
-                                                ops.mixer_norm, eps=config.eps))
-            launches.append(self._gemm_tile("gemm_tile_store", ops.entry, self.mixer_in_tile, qkv))
-            launches.append(self._quantize_tile("quantize_tile_plain", values, hidden, qkv))
-            launches.append(self._gemm_tile("gemm_tile_residual", ops.out, self.residual_tile, hidden))
-            launches.append(self._quantize_tile("quantize_tile_norm", self.residual_tile, hidden, hidden,
-                                                ops.ffn_norm, eps=config.eps))
-            launches.append(self._gemm_tile("gemm_tile_silu_pair", ops.gate_up, self.ffn_tile, dense))
-            launches.append(self._quantize_tile("quantize_tile_plain", self.ffn_tile, dense, dense))
-            launches.append(self._gemm_tile("gemm_tile_residual", ops.down, self.residual_tile, hidden))
-        launches.append(Launch(self.module.kernel("gather_token"), ((hidden + THREADS - 1) // THREADS, 1, 1),
-                               (THREADS, 1, 1),
-                               [pointer(self.residual_tile), pointer(self.residual), int32(hidden),
-                                pointer(self.tile_valid)]))
-        return launches
+            steps.append(self._quantize_tile(MODE_NORM, self.residual_tile, hidden, hidden, ops.mixer_norm, config.eps))
+            steps.append(self._gemm_tile("gemm_tile_store", ops.entry, self.mixer_in_tile, qkv))
+            steps.append(self._quantize_tile(MODE_PLAIN, values, hidden, qkv))
+            steps.append(self._gemm_tile("gemm_tile_residual", ops.out, self.residual_tile, hidden))
+            steps.append(self._quantize_tile(MODE_NORM, self.residual_tile, hidden, hidden, ops.ffn_norm, config.eps))
+            steps.append(self._gemm_tile("gemm_tile_silu_pair", ops.gate_up, self.ffn_tile, dense))
+            steps.append(self._quantize_tile(MODE_PLAIN, self.ffn_tile, dense, dense))
+            steps.append(self._gemm_tile("gemm_tile_residual", ops.down, self.residual_tile, hidden))
+        gather = Launch(self.module.kernel("gather_token"), (blocks, 1, 1), (THREADS, 1, 1),
+                        [pointer(self.residual_tile), pointer(self.residual), int32(hidden),
+                         pointer(self.tile_valid)])
+        return {tokens: [*(step(tokens) for step in steps), gather] for tokens in TILES}
 
     # ------------------------------------------------------------------ running
 
@@ -270,26 +283,28 @@ class StackDecoder:
 
     @torch.no_grad()
     def prefill(self, input_ids) -> torch.Tensor:
-        """Runs the prompt in 32-token tiles (kernel_decoder.py:456-479), then the head on its last token:
-        the logits are left in ``self.logits`` and the first token (greedy, or drawn by the sampler) in
-        the ring's last slot."""
-        ids = torch.as_tensor(input_ids, dtype=torch.int64).reshape(-1)
+        """Runs the prompt in tiles (kernel_decoder.py:456-479), each the smallest of TILES that holds the
+        tokens left, then the head on its last token: the logits are left in ``self.logits`` and the first
+        token (greedy, or drawn by the sampler) in the ring's last slot."""
+        ids = torch.as_tensor(input_ids, dtype=torch.int64).reshape(-1).cpu()
         length = int(ids.numel())
         if length == 0:
             raise ValueError("the prompt must not be empty")
         if int(ids.min()) < 0 or int(ids.max()) >= self.config.vocab:
             raise IndexError(f"token id is out of range for vocab_size={self.config.vocab}")
-        ids = ids.to(self.device)
-        for start in range(0, length, TILE):
-            chunk = ids[start:start + TILE]
-            count = int(chunk.numel())
-            self.tile_tokens.zero_()
-            self.tile_tokens[:count].copy_(chunk)
-            self.tile_valid.fill_(count)
+        host, start = self._tile_host, 0
+        while start < length:
+            count = min(length - start, TILES[-1])
+            tokens = next(size for size in TILES if size >= count)
+            host[0] = count
+            host[1:1 + count] = ids[start:start + count]
+            host[1 + count:1 + tokens] = 0
+            self.tile_input[:1 + tokens].copy_(host[:1 + tokens])
             if self._tile_graph is not None:
-                self._tile_graph.replay()  # one replay per tile (kernel_decoder.py:444-447)
+                self._tile_graph[tokens].replay()  # one replay per tile (kernel_decoder.py:444-447)
             else:
-                self._run(self._tile)
+                self._run(self._tiles[tokens])
+            start += count
         self._run(self._first)
         self.position = 0
         return self.logits
@@ -304,10 +319,10 @@ class StackDecoder:
     def capture(self) -> bool:
         """Records one burst of decode steps into a HIP graph (kernel_decoder.py:694-719).  With sampling,
         the uniforms are drawn inside the graph, fresh on every replay; the sampler's `seen` is restored
-        after the warm-up and the capture, as the ring is.  Then records the prefill tile program as a
-        second graph (kernel_decoder.py:482-509), which prefill() replays once per 32-token tile after
+        after the warm-up and the capture, as the ring is.  Then records the prefill tile program of every
+        tile size as a graph (kernel_decoder.py:482-509), which prefill() replays once per tile after
         filling the device buffers tile_tokens and tile_valid; the residual the last prefill left is
-        restored after its warm-up and capture."""
+        restored after their warm-up and capture."""
         if self.position % self.burst != 0:
             raise KernelError("capture at a burst boundary")
         saved = self.history.clone()
@@ -331,24 +346,26 @@ class StackDecoder:
         if seen is not None:
             self.sampler.seen.copy_(seen)
         self._graph = graph
-        self._tile_graph = self._capture_tile(stream)
+        self._tile_graph = self._capture_tiles(stream)
         return True
 
-    def _capture_tile(self, stream: torch.cuda.Stream) -> torch.cuda.CUDAGraph:
+    def _capture_tiles(self, stream: torch.cuda.Stream) -> dict[int, torch.cuda.CUDAGraph]:
         residual, valid = self.residual.clone(), self.tile_valid.clone()
         self.tile_valid.fill_(TILE)
         stream.wait_stream(torch.cuda.current_stream(self.device))
         with torch.cuda.stream(stream):
-            self._run(self._tile)
+            self._run(self._tiles[TILE])
         torch.cuda.current_stream(self.device).wait_stream(stream)
         torch.cuda.synchronize(self.device)
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=stream):
-            self._run(self._tile)
+        graphs = {}
+        for tokens, launches in self._tiles.items():
+            graphs[tokens] = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graphs[tokens], stream=stream):
+                self._run(launches)
         torch.cuda.synchronize(self.device)
         self.residual.copy_(residual)
         self.tile_valid.copy_(valid)
-        return graph
+        return graphs
 
     @torch.no_grad()
     def advance_many(self, count: int) -> list[int]:
