@@ -186,6 +186,22 @@ hipError_t gemm_tile_store_wide(hipStream_t stream, IVONAR_GEMM_ARGS);
 hipError_t gemm_tile_residual_wide(hipStream_t stream, IVONAR_GEMM_ARGS);
 hipError_t gemm_tile_silu_pair_wide(hipStream_t stream, IVONAR_GEMM_ARGS);
 
+/* A whole linear layer (no reference counterpart as one call; the forward of
+ * quantization.py:177-178): output fp32 [m, rows] from m contiguous rows of n
+ * inputs of type dtype (0 fp32, 1 fp16, 2 bfloat16; the half types are converted
+ * exactly as they are read).  Up to two launches: gemv_plain_store for one
+ * fp32 row, else ivonar_quantize_rows and gemm_tile_store (one row:
+ * gemv_prequant_store), with their results and rules.  work: 16-byte aligned, m
+ * * (ceil(n/64) * 68 + 4) bytes, not read before they are written; NULL for
+ * one fp32 row. */
+hipError_t ivonar_linear(hipStream_t stream, const void* input, int dtype, int m, void* work, const uint8_t* packed,
+                         const uint16_t* scales, const float* bias, float* output, int rows, int n, int row_bytes,
+                         int groups);
+/* 1 if ivonar_linear takes half rows of n inputs at this address (n up to 8192,
+ * or up to 32768 if n is a multiple of 4 and the address one of 8), else 0.
+ * Host only. */
+int ivonar_linear_half(int n, const void* input);
+
 /* ------------------------------------------------------------- embedding */
 
 /* ternary.cu:411-419: output[i] = (code[token, i] - 1) * scale[token, i/128]. */

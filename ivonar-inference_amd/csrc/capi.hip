@@ -153,7 +153,8 @@ hipError_t static_scratch(Scratch** out) {
 }
 
 hipError_t quant_entry(hipStream_t stream, int mode, const float* input, int in_stride, const float* aux, int n,
-                       float eps, int splits, int m, int8_t* q8_out, int32_t* xsum_out, float* scale_out) {
+                       float eps, int splits, int m, int8_t* q8_out, int32_t* xsum_out, float* scale_out,
+                       int dtype = kFloat32) {
   if (n <= 0 || m < 0 || input == nullptr || q8_out == nullptr || xsum_out == nullptr || scale_out == nullptr)
     return hipErrorInvalidValue;
   if (!aligned16(q8_out) || ((uintptr_t)xsum_out & 3u) != 0) return hipErrorInvalidValue;
@@ -163,7 +164,7 @@ hipError_t quant_entry(hipStream_t stream, int mode, const float* input, int in_
   if (mode < kPlain || mode > kAttn) return hipErrorInvalidValue;
   if (m > 1 && in_stride < (mode == kAttn ? 1 : n)) return hipErrorInvalidValue;
   QuantArgs q{mode, input, in_stride, aux, n, eps, splits > 0 ? splits : 1, head_dim, m,
-              q8_out, xsum_out, scale_out};
+              q8_out, xsum_out, scale_out, false, dtype};
   return launch_quantize(stream, q);
 }
 
@@ -414,6 +415,32 @@ hipError_t gemm_tile_silu_pair_wide(hipStream_t stream, IVONAR_GEMM_ARGS) {
   (void)lanes;
   return GEMM_PASS_ENTRY(kSiluPair);
 }
+
+hipError_t ivonar_linear(hipStream_t stream, const void* input, int dtype, int m, void* work, const uint8_t* packed,
+                         const uint16_t* scales, const float* bias, float* output, int rows, int n, int row_bytes,
+                         int groups) {
+  const float* x = static_cast<const float*>(input);
+  if (m == 1 && dtype == kFloat32)
+    return gemv_entry(stream, kPlain, kStore, false, x, nullptr, nullptr, nullptr, nullptr, packed, scales, bias,
+                      output, rows, n, row_bytes, groups, 1, 0.0f);
+  // Everything the second launch would refuse is refused before the first one goes out.
+  hipError_t status = check_matrix(packed, scales, rows, n, row_bytes, groups);
+  if (status != hipSuccess) return status;
+  if (dtype < kFloat32 || dtype > kBfloat16 || m < 0 || work == nullptr || output == nullptr)
+    return hipErrorInvalidValue;
+  const size_t chunks = (size_t)ceil_div(n, kChunk);
+  int8_t* q8 = static_cast<int8_t*>(work);
+  int32_t* xsum = reinterpret_cast<int32_t*>(q8 + (size_t)m * chunks * kChunk);
+  float* scale = reinterpret_cast<float*>(xsum + (size_t)m * chunks);
+  status = quant_entry(stream, kPlain, x, n, nullptr, n, 0.0f, 1, m, q8, xsum, scale, dtype);
+  if (status != hipSuccess) return status;
+  if (m == 1)
+    return gemv_entry(stream, kPlain, kStore, true, nullptr, nullptr, q8, xsum, scale, packed, scales, bias, output,
+                      rows, n, row_bytes, groups, 1, 0.0f);
+  return gemm_entry(stream, kStore, q8, xsum, scale, packed, scales, bias, output, rows, n, row_bytes, groups, rows,
+                    m);
+}
+int ivonar_linear_half(int n, const void* input) { return n > 0 && quantize_half_applies(n, input) ? 1 : 0; }
 
 hipError_t embed_token(hipStream_t stream, const int64_t* token, const uint8_t* packed, const uint16_t* scales,
                        float* output, int n, int row_bytes, int groups) {

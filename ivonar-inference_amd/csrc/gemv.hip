@@ -254,7 +254,7 @@ __global__ __launch_bounds__(block_threads<ROLL>()) void gemv_kernel(GemvPtrs in
       auto quantize = [&](auto nb_c) {
         constexpr int NB = decltype(nb_c)::value;
         if (vec) return quantize_plain_row4_to_lds<NB>(src, chunks, q, slots, first_loads);
-        return quantize_row_to_lds<MODE, NB>(src, chunks, q, slots, first_loads);
+        return quantize_row_to_lds<MODE, NB, float>(src, chunks, q, slots, first_loads);
       };
       if constexpr (LANES == 64) sx = quantize(std::integral_constant<int, kBatch>{});
       else if (sh.n <= 4 * kThreads) sx = quantize(std::integral_constant<int, 4>{});

@@ -51,6 +51,8 @@ constexpr long long kTokenPartialFloats = 4LL << 20;
 hipError_t scratch_for_stream(hipStream_t stream, Scratch** out);
 hipError_t init_device(int device);
 
+enum Dtype : int { kFloat32 = 0, kFloat16 = 1, kBfloat16 = 2 };
+
 struct QuantArgs {
   int mode;
   const float* input;
@@ -67,8 +69,13 @@ struct QuantArgs {
   // Write each quad in the nibble-split form the 4-bit GEMV reads (split_quad_word)
   // instead of q8 bytes; the chunk sums and the scale are the same.
   bool split = false;
+  // Type of the input values (PLAIN rows only for the half types, which are
+  // converted exactly as they are read).
+  int dtype = kFloat32;
 };
 hipError_t launch_quantize(hipStream_t stream, const QuantArgs& a);
+// Whether launch_quantize takes PLAIN half rows of n inputs at this address.
+bool quantize_half_applies(int n, const void* input);
 
 struct GemvArgs {
   int mode;    // kPlain / kNorm / kAttn (ignored when q8_in is set)

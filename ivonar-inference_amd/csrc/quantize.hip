@@ -85,14 +85,15 @@ __device__ __forceinline__ float block_absmax(float v, float* slots) {
 // once into registers (quantize_row_to_lds: the reference's order of the sum
 // of squares), the q8 bytes are exchanged through LDS, and thread w writes the
 // q8 words w + 256 i.
-template <int MODE, int NB>
+template <int MODE, int NB, typename In>
 __global__ __launch_bounds__(kThreads) void quantize_row_kernel(QuantArgs a) {
   __shared__ float slots[64];
   __shared__ __align__(16) unsigned char lds_q[NB * kThreads];
   const int t = blockIdx.y;
   const int chunks = (a.n + kChunk - 1) / kChunk;
-  const RowSource src{a.input + (size_t)t * a.in_stride, a.aux, a.n, a.eps, a.splits, a.head_dim};
-  const float scale = quantize_row_to_lds<MODE, NB>(src, chunks, lds_q, slots);
+  const In* row = reinterpret_cast<const In*>(a.input) + (size_t)t * a.in_stride;
+  const RowSource src{reinterpret_cast<const float*>(row), a.aux, a.n, a.eps, a.splits, a.head_dim};
+  const float scale = quantize_row_to_lds<MODE, NB, In>(src, chunks, lds_q, slots);
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < NB / 4; ++i) {
@@ -169,23 +170,23 @@ __global__ __launch_bounds__(T) void quantize_norm4_kernel(QuantArgs a) {
 }
 
 // 16-byte aligned PLAIN rows of up to 4 * T * NC inputs: thread t holds the
-// float4 t + T c, whose four int8 values become word j = t & 3 of the quad
+// float4 t + T c (of the values, four halves in the half types), whose four int8 values become word j = t & 3 of the quad
 // after a byte transpose over its four lanes; word f of the row is then the
 // thread's own, so the stores are as contiguous as the loads.  SLICED (few
 // long rows): NC blocks per row, each of which takes the absmax of the whole
 // row and quantizes one float4 per thread.
-template <int T, int NC, bool SLICED>
+template <int T, int NC, bool SLICED, typename In>
 __global__ __launch_bounds__(T) void quantize_plain_kernel(QuantArgs a) {
   __shared__ float slots[T / 64];
   const int t = blockIdx.y, tid = threadIdx.x;
   const int chunks = (a.n + kChunk - 1) / kChunk;
   const int n4 = a.n >> 2;
-  const float4* row = reinterpret_cast<const float4*>(a.input + (size_t)t * a.in_stride);
+  const In* row = reinterpret_cast<const In*>(a.input) + (size_t)t * a.in_stride;
   float4 v[NC];
 #pragma unroll
-  for (int c = 0; c < NC; ++c) v[c] = row[min(c * T + tid, n4 - 1)];
+  for (int c = 0; c < NC; ++c) v[c] = load4(row, min(c * T + tid, n4 - 1));
   float4 mine;
-  if constexpr (SLICED) mine = row[min((int)blockIdx.x * T + tid, n4 - 1)];
+  if constexpr (SLICED) mine = load4(row, min((int)blockIdx.x * T + tid, n4 - 1));
   float amax = 0.0f;
 #pragma unroll
   for (int c = 0; c < NC; ++c)
@@ -297,13 +298,13 @@ __global__ __launch_bounds__(T) void quantize_attn_kernel(QuantArgs a) {
   if (tid == 0) a.scale[t] = scale;
 }
 
-template <int MODE>
+template <int MODE, typename In = float>
 bool launch_row(hipStream_t stream, const QuantArgs& a) {
   const dim3 grid(1, a.m), block(kThreads);
-  if (a.n <= 4 * kThreads) hipLaunchKernelGGL((quantize_row_kernel<MODE, 4>), grid, block, 0, stream, a);
-  else if (a.n <= 8 * kThreads) hipLaunchKernelGGL((quantize_row_kernel<MODE, 8>), grid, block, 0, stream, a);
-  else if (a.n <= 16 * kThreads) hipLaunchKernelGGL((quantize_row_kernel<MODE, 16>), grid, block, 0, stream, a);
-  else if (a.n <= 32 * kThreads) hipLaunchKernelGGL((quantize_row_kernel<MODE, 32>), grid, block, 0, stream, a);
+  if (a.n <= 4 * kThreads) hipLaunchKernelGGL((quantize_row_kernel<MODE, 4, In>), grid, block, 0, stream, a);
+  else if (a.n <= 8 * kThreads) hipLaunchKernelGGL((quantize_row_kernel<MODE, 8, In>), grid, block, 0, stream, a);
+  else if (a.n <= 16 * kThreads) hipLaunchKernelGGL((quantize_row_kernel<MODE, 16, In>), grid, block, 0, stream, a);
+  else if (a.n <= 32 * kThreads) hipLaunchKernelGGL((quantize_row_kernel<MODE, 32, In>), grid, block, 0, stream, a);
   else return false;
   return true;
 }
@@ -329,26 +330,27 @@ bool launch_norm(hipStream_t stream, const QuantArgs& a, bool aligned) {
   return true;
 }
 
-template <int T, int NC>
+template <int T, int NC, typename In>
 void launch_plain_shape(hipStream_t stream, const QuantArgs& a) {
   // Few long rows: one CU would spend more time on a row's conversions than on
   // its absmax (12 rows of 28672: 5.4 us with one block per row, 3.5 with eight).
   if (NC > 1 && (long long)a.m * NC <= 2LL * device_cus())
-    hipLaunchKernelGGL((quantize_plain_kernel<T, NC, (NC > 1)>), dim3(NC, a.m), dim3(T), 0, stream, a);
+    hipLaunchKernelGGL((quantize_plain_kernel<T, NC, (NC > 1), In>), dim3(NC, a.m), dim3(T), 0, stream, a);
   else
-    hipLaunchKernelGGL((quantize_plain_kernel<T, NC, false>), dim3(1, a.m), dim3(T), 0, stream, a);
+    hipLaunchKernelGGL((quantize_plain_kernel<T, NC, false, In>), dim3(1, a.m), dim3(T), 0, stream, a);
 }
 
+template <typename In>
 bool launch_plain(hipStream_t stream, const QuantArgs& a) {
   const int n4 = a.n >> 2;
   const bool many = a.m >= kManyRows;
-  if (n4 <= 256) launch_plain_shape<256, 1>(stream, a);
-  else if (n4 <= 1024 && many) launch_plain_shape<256, 4>(stream, a);
-  else if (n4 <= 1024) launch_plain_shape<1024, 1>(stream, a);
-  else if (n4 <= 2048 && many) launch_plain_shape<512, 4>(stream, a);
-  else if (n4 <= 2048) launch_plain_shape<1024, 2>(stream, a);
-  else if (n4 <= 4096) launch_plain_shape<1024, 4>(stream, a);
-  else if (n4 <= 8192) launch_plain_shape<1024, 8>(stream, a);
+  if (n4 <= 256) launch_plain_shape<256, 1, In>(stream, a);
+  else if (n4 <= 1024 && many) launch_plain_shape<256, 4, In>(stream, a);
+  else if (n4 <= 1024) launch_plain_shape<1024, 1, In>(stream, a);
+  else if (n4 <= 2048 && many) launch_plain_shape<512, 4, In>(stream, a);
+  else if (n4 <= 2048) launch_plain_shape<1024, 2, In>(stream, a);
+  else if (n4 <= 4096) launch_plain_shape<1024, 4, In>(stream, a);
+  else if (n4 <= 8192) launch_plain_shape<1024, 8, In>(stream, a);
   else return false;
   return true;
 }
@@ -377,13 +379,26 @@ bool launch_attn(hipStream_t stream, const QuantArgs& a) {
 
 }  // namespace
 
+bool quantize_half_applies(int n, const void* input) {
+  return (n & 3) == 0 && (reinterpret_cast<uintptr_t>(input) & 7) == 0 ? n <= 32768 : n <= 32 * kThreads;
+}
+
 hipError_t launch_quantize(hipStream_t stream, const QuantArgs& a) {
   if (a.m <= 0) return hipSuccess;
+  if (a.dtype != kFloat32) {
+    if (a.mode != kPlain || a.n <= 0 || !quantize_half_applies(a.n, a.input)) return hipErrorInvalidValue;
+    const bool aligned = (a.n & 3) == 0 && (a.in_stride & 3) == 0 && (reinterpret_cast<uintptr_t>(a.input) & 7) == 0;
+    bool launched = false;
+    if (a.dtype == kFloat16) launched = aligned ? launch_plain<Half>(stream, a) : launch_row<kPlain, Half>(stream, a);
+    if (a.dtype == kBfloat16)
+      launched = aligned ? launch_plain<Bfloat>(stream, a) : launch_row<kPlain, Bfloat>(stream, a);
+    return launched ? hipGetLastError() : hipErrorInvalidValue;
+  }
   const int chunks = ceil_div(a.n, kChunk);
   const bool aligned = (a.n & 3) == 0 && (a.in_stride & 3) == 0 && (reinterpret_cast<uintptr_t>(a.input) & 15) == 0;
   bool launched = false;
   switch (a.mode) {
-    case kPlain: launched = aligned ? launch_plain(stream, a) : launch_row<kPlain>(stream, a); break;
+    case kPlain: launched = aligned ? launch_plain<float>(stream, a) : launch_row<kPlain>(stream, a); break;
     case kNorm: launched = launch_norm(stream, a, aligned); break;
     case kAttn: launched = launch_attn(stream, a); break;
     default: return hipErrorInvalidValue;

@@ -40,6 +40,26 @@ __device__ __forceinline__ float h2f(uint16_t bits) {
   return (float)h;
 }
 
+// Activations a row may be stored in.
+struct Half {
+  uint16_t bits;
+};
+struct Bfloat {
+  uint16_t bits;
+};
+__device__ __forceinline__ float to_float(float v) { return v; }
+__device__ __forceinline__ float to_float(Half v) { return h2f(v.bits); }
+__device__ __forceinline__ float to_float(Bfloat v) { return __uint_as_float((unsigned)v.bits << 16); }
+
+// Inputs 4i .. 4i + 3 of a row: one 16-byte load, or one of 8 bytes for the half types.
+__device__ __forceinline__ float4 load4(const float* row, int i) { return reinterpret_cast<const float4*>(row)[i]; }
+template <typename In>
+__device__ __forceinline__ float4 load4(const In* row, int i) {
+  const uint2 v = reinterpret_cast<const uint2*>(row)[i];
+  return float4{to_float(In{(uint16_t)v.x}), to_float(In{(uint16_t)(v.x >> 16)}), to_float(In{(uint16_t)v.y}),
+                to_float(In{(uint16_t)(v.y >> 16)})};
+}
+
 // exp(x): Cody-Waite reduction x = n*ln2 + r, degree-7 Taylor polynomial of
 // e^r in Horner form, scaling by 2^n in two exact steps.  Every operation is
 // an explicit IEEE fp32 op, so the CPU oracle reproduces it bit for bit.
@@ -479,7 +499,7 @@ struct NoLoads {
   __device__ void operator()() const {}
 };
 
-template <int MODE, int NB = kBatch, typename AfterLoads = NoLoads>
+template <int MODE, int NB = kBatch, typename In = float, typename AfterLoads = NoLoads>
 __device__ __forceinline__ float quantize_row_to_lds(const RowSource& src, int chunks, unsigned char* lds_q,
                                                      float* slots, AfterLoads after_loads = AfterLoads{}) {
   static_assert(MODE == kPlain || MODE == kNorm, "register path for PLAIN and NORM rows");
@@ -490,7 +510,7 @@ __device__ __forceinline__ float quantize_row_to_lds(const RowSource& src, int c
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
     const int i = min(b * kThreads + tid, n - 1);
-    v[b] = src.input[i];
+    v[b] = to_float(reinterpret_cast<const In*>(src.input)[i]);
     w[b] = MODE == kNorm ? src.aux[i] : 1.0f;
   }
   // Loads the caller issues behind the row's (loads return in order, so the

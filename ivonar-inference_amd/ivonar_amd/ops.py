@@ -9,7 +9,7 @@ the current stream and never synchronises.  The shapes follow the reference:
 * ``gemv(matrix, x [K])`` -> y [N]: the decode GEMV (M = 1);
 * ``gemm(matrix, q8, xsum, scale)`` -> y [M, N]: int8 MFMA over M tokens;
 * ``ternary_linear(x [..., K], matrix)`` -> [..., N]: GEMV for one token,
-  quantize + MFMA GEMM otherwise;
+  quantize + MFMA GEMM otherwise, of fp32, fp16 or bfloat16 rows;
 * ``group_partials(matrix, q8, xsum)`` -> int32 [N, G]: the GEMV's exact
   per-128-group partial sums (test export).
 """
@@ -32,6 +32,7 @@ _GEMV_NAMES = {
     ("norm", "silu_pair"): "gemv_norm_silu_pair",
     ("attn", "residual"): "gemv_attn_residual",
 }
+_LINEAR_DTYPES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 _GEMM_NAMES = {"store": "gemm_tile_store", "residual": "gemm_tile_residual", "silu_pair": "gemm_tile_silu_pair"}
 
 
@@ -40,7 +41,7 @@ def _require_device(*tensors: Tensor | None) -> torch.device:
     for tensor in tensors:
         if tensor is None:
             continue
-        if tensor.device.type != "cuda":
+        if not tensor.is_cuda:
             raise KernelError("ternary kernels need tensors on a ROCm device")
         if device is None:
             device = tensor.device
@@ -48,6 +49,18 @@ def _require_device(*tensors: Tensor | None) -> torch.device:
         raise KernelError("no device tensor given")
     initialise(device.index if device.index is not None else torch.cuda.current_device())
     return device
+
+
+def _address(tensor: Tensor | None) -> int | None:
+    return None if tensor is None else tensor.data_ptr()
+
+
+def _call(name: str, device: torch.device, *args) -> None:
+    """One entry point on the device's current stream; the arguments are plain ints and floats, which ctypes
+    converts by the entry point's signature (building ctypes objects first costs as much as the launch)."""
+    status = getattr(library(), name)(current_stream(device), *args)
+    if status != 0:
+        check(status, name)
 
 
 def activation_buffers(m: int, n: int, device: torch.device) -> tuple[Tensor, Tensor, Tensor]:
@@ -71,13 +84,8 @@ def quantize_rows(
     m = rows.shape[0]
     width = int(n if n is not None else rows.shape[1])
     q8, xsum, scale = out if out is not None else activation_buffers(m, width, device)
-    check(
-        library().ivonar_quantize_rows(
-            current_stream(device), mode, pointer(rows), int32(rows.stride(0)), pointer(aux), int32(width),
-            float32(eps), int32(splits), int32(m), pointer(q8), pointer(xsum), pointer(scale),
-        ),
-        "ivonar_quantize_rows",
-    )
+    _call("ivonar_quantize_rows", device, int(mode), rows.data_ptr(), rows.stride(0), _address(aux), width, float(eps),
+          int(splits), m, q8.data_ptr(), xsum.data_ptr(), scale.data_ptr())
     return q8, xsum, scale
 
 
@@ -98,16 +106,9 @@ def gemv(
         if epilogue == "residual":
             raise KernelError("a residual GEMV needs the output tensor it adds into")
         out = torch.empty(rows_out, dtype=torch.float32, device=device)
-    function = getattr(library(), name)
-    check(
-        function(
-            current_stream(device), pointer(x), pointer(aux), pointer(None), pointer(None), pointer(None),
-            pointer(matrix.packed), pointer(matrix.scales), pointer(matrix.bias), pointer(out),
-            int32(matrix.rows), int32(matrix.in_features), int32(matrix.row_bytes), int32(matrix.groups),
-            int32(matrix.lanes), int32(splits), float32(eps), pointer(None), int32(0),
-        ),
-        name,
-    )
+    _call(name, device, x.data_ptr(), _address(aux), None, None, None, matrix.packed.data_ptr(),
+          matrix.scales.data_ptr(), _address(matrix.bias), out.data_ptr(), matrix.rows, matrix.in_features,
+          matrix.row_bytes, matrix.groups, matrix.lanes, int(splits), float(eps), None, 0)
     return out
 
 
@@ -142,15 +143,9 @@ def gemm(
         out = torch.empty((rows, width), dtype=torch.float32, device=device)
     stride = int(out_stride if out_stride is not None else (out.stride(0) if out.ndim == 2 else width))
     name = _GEMM_NAMES[epilogue]
-    check(
-        getattr(library(), name)(
-            current_stream(device), pointer(q8), pointer(xsum), pointer(scale), pointer(matrix.packed),
-            pointer(matrix.scales), pointer(matrix.bias), pointer(out), int32(matrix.rows),
-            int32(matrix.in_features), int32(matrix.row_bytes), int32(matrix.groups), int32(matrix.lanes),
-            int32(stride), int32(rows),
-        ),
-        name,
-    )
+    _call(name, device, q8.data_ptr(), xsum.data_ptr(), scale.data_ptr(), matrix.packed.data_ptr(),
+          matrix.scales.data_ptr(), _address(matrix.bias), out.data_ptr(), matrix.rows, matrix.in_features,
+          matrix.row_bytes, matrix.groups, matrix.lanes, stride, rows)
     return out
 
 
@@ -196,16 +191,24 @@ def argmax(values: Tensor, out: Tensor | None = None) -> Tensor:
 
 
 def ternary_linear(x: Tensor, matrix: Matrix) -> Tensor:
-    """y = ternary linear layer of x [..., K] (GEMV for one token, MFMA GEMM otherwise)."""
+    """y = ternary linear layer of x [..., K] (GEMV for one token, MFMA GEMM otherwise), one native call; half
+    rows are converted as the quantizer reads them, other types and strided inputs before it."""
     device = _require_device(x, matrix.packed)
-    if x.shape[-1] != matrix.in_features:
-        raise KernelError(f"input width {x.shape[-1]} does not match the layer's {matrix.in_features}")
+    width = matrix.in_features
+    if x.shape[-1] != width:
+        raise KernelError(f"input width {x.shape[-1]} does not match the layer's {width}")
     lead = x.shape[:-1]
-    rows = x.reshape(-1, matrix.in_features).float().contiguous()
-    m = rows.shape[0]
-    if m == 1:
-        return gemv(matrix, rows[0]).reshape(*lead, matrix.rows)
-    q8, xsum, scale = quantize_rows(rows)
-    out = torch.empty((m, matrix.rows), dtype=torch.float32, device=device)
-    gemm(matrix, q8, xsum, scale, out=out)
-    return out.reshape(*lead, matrix.rows)
+    rows = x if x.is_contiguous() else x.reshape(-1, width).contiguous()
+    dtype = _LINEAR_DTYPES.get(rows.dtype)
+    if dtype is None or (dtype != 0 and not library().ivonar_linear_half(width, rows.data_ptr())):
+        rows, dtype = rows.float(), 0
+    m = rows.numel() // width
+    out = torch.empty((*lead, matrix.rows), dtype=torch.float32, device=device)
+    work = None
+    if m != 1 or dtype != 0:
+        # q8 rows, chunk sums and token scales of the call
+        work = torch.empty(m * (-(-width // CHUNK) * (CHUNK + 4) + 4), dtype=torch.uint8, device=device)
+    _call("ivonar_linear", device, rows.data_ptr(), dtype, m, _address(work), matrix.packed.data_ptr(),
+          matrix.scales.data_ptr(), _address(matrix.bias), out.data_ptr(), matrix.rows, width, matrix.row_bytes,
+          matrix.groups)
+    return out

@@ -99,7 +99,7 @@ class TernaryLinear(nn.Module):
         """The device-resident, row-padded kernel operand of this layer (built once)."""
         from .matrix import Matrix
 
-        device = self.packed_weight.device
+        device = self._buffers["packed_weight"].device
         if self._matrix is None or self._matrix.packed.device != device:
             self._matrix = Matrix([self], device)
         return self._matrix

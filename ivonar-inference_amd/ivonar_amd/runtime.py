@@ -62,6 +62,7 @@ SIGNATURES: dict[str, list] = {
         "gemm_tile_store", "gemm_tile_residual", "gemm_tile_silu_pair", "gemm_tile_store_wide",
         "gemm_tile_residual_wide", "gemm_tile_silu_pair_wide",
     )},
+    "ivonar_linear": [_P, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I],
     "embed_token": [_P, _P, _P, _P, _I, _I, _I],
     "embed_tile": [_P, _P, _P, _P, _I, _I, _I, _I],
     "gather_token": [_P, _P, _I, _P],
@@ -83,6 +84,8 @@ _modules: dict[tuple, "Module"] = {}
 def library() -> ctypes.CDLL:
     """Load the HIP library once (after torch, so it binds torch's HIP runtime)."""
     global _library
+    if _library is not None:
+        return _library
     with _lock:
         if _library is None:
             if not LIBRARY.is_file():
@@ -106,6 +109,8 @@ def library() -> ctypes.CDLL:
             lib.ivonar_gemm_plan.restype = c_int
             lib.ivonar_stream_read_sink_words.argtypes = []
             lib.ivonar_stream_read_sink_words.restype = c_int
+            lib.ivonar_linear_half.argtypes = [c_int, c_void_p]
+            lib.ivonar_linear_half.restype = c_int
             lib.ivonar_token_finish_limit.argtypes = [c_int]
             lib.ivonar_token_finish_limit.restype = c_int
             for name, argtypes in SIGNATURES.items():
@@ -136,9 +141,8 @@ def gemm_plan(m: int, rows: int, n: int) -> int:
 
 def initialise(device_index: int) -> None:
     """Allocate the library's per-device scratch (outside any graph capture)."""
-    with _lock:
-        if device_index in _initialised:
-            return
+    if device_index in _initialised:
+        return
     current = torch.cuda.current_device()
     if current != device_index:
         torch.cuda.set_device(device_index)
@@ -279,7 +283,9 @@ def float32(value: float) -> c_float:
 
 
 def current_stream(device: torch.device | None = None) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    index = None if device is None else device.index
+    # The stream's handle alone: torch.cuda.current_stream() builds a Stream object around it.
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 class Driver:
