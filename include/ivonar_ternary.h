@@ -186,17 +186,31 @@ hipError_t gemm_tile_store_wide(hipStream_t stream, IVONAR_GEMM_ARGS);
 hipError_t gemm_tile_residual_wide(hipStream_t stream, IVONAR_GEMM_ARGS);
 hipError_t gemm_tile_silu_pair_wide(hipStream_t stream, IVONAR_GEMM_ARGS);
 
+/* gemm_tile_* with the epilogue as an argument (0 store, 1 residual, 2 silu
+ * pair) and a workspace: with work 16-byte aligned and work_bytes at least
+ * ivonar_gemm_work(m, rows, n), and that not 0, the long-prompt kernel on the
+ * block-scaled MFMA runs (the same results bit for bit); else gemm_tile_*.
+ * The workspace is written before it is read and free again once the call has
+ * run. */
+long long ivonar_gemm_work(int m, int rows, int n);
+hipError_t ivonar_gemm(hipStream_t stream, int epilogue, const int8_t* q8_in, const int32_t* xsum_in,
+                       const float* scale_in, const uint8_t* packed, const uint16_t* scales, const float* bias,
+                       float* output, int rows, int n, int row_bytes, int groups, int out_stride, int m, void* work,
+                       long long work_bytes);
+
 /* A whole linear layer (no reference counterpart as one call; the forward of
  * quantization.py:177-178): output fp32 [m, rows] from m contiguous rows of n
  * inputs of type dtype (0 fp32, 1 fp16, 2 bfloat16; the half types are converted
- * exactly as they are read).  Up to two launches: gemv_plain_store for one
- * fp32 row, else ivonar_quantize_rows and gemm_tile_store (one row:
- * gemv_prequant_store), with their results and rules.  work: 16-byte aligned, m
- * * (ceil(n/64) * 68 + 4) bytes, not read before they are written; NULL for
- * one fp32 row. */
-hipError_t ivonar_linear(hipStream_t stream, const void* input, int dtype, int m, void* work, const uint8_t* packed,
-                         const uint16_t* scales, const float* bias, float* output, int rows, int n, int row_bytes,
-                         int groups);
+ * exactly as they are read).  gemv_plain_store for one fp32 row, else
+ * ivonar_quantize_rows and ivonar_gemm (one row: gemv_prequant_store), with
+ * their results and rules.  work: 16-byte aligned, ivonar_linear_work bytes
+ * (host only; 0: may be NULL), written before they are read.  With fewer, at
+ * least m * (ceil(n/64) * 68 + 4) rounded up to 16, the GEMM runs without a
+ * workspace. */
+long long ivonar_linear_work(int dtype, int m, int rows, int n);
+hipError_t ivonar_linear(hipStream_t stream, const void* input, int dtype, int m, void* work, long long work_bytes,
+                         const uint8_t* packed, const uint16_t* scales, const float* bias, float* output, int rows,
+                         int n, int row_bytes, int groups);
 /* 1 if ivonar_linear takes half rows of n inputs at this address (n up to 8192,
  * or up to 32768 if n is a multiple of 4 and the address one of 8), else 0.
  * Host only. */

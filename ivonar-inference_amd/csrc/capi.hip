@@ -170,7 +170,8 @@ hipError_t quant_entry(hipStream_t stream, int mode, const float* input, int in_
 
 hipError_t gemm_entry(hipStream_t stream, int epi, const int8_t* q8_in, const int32_t* xsum_in,
                       const float* scale_in, const uint8_t* packed, const uint16_t* scales, const float* bias,
-                      float* output, int rows, int n, int row_bytes, int groups, int out_stride, int m) {
+                      float* output, int rows, int n, int row_bytes, int groups, int out_stride, int m,
+                      void* work = nullptr, long long work_bytes = 0) {
   hipError_t status = check_matrix(packed, scales, rows, n, row_bytes, groups);
   if (status != hipSuccess) return status;
   if (m < 0 || q8_in == nullptr || xsum_in == nullptr || scale_in == nullptr || output == nullptr)
@@ -180,6 +181,10 @@ hipError_t gemm_entry(hipStream_t stream, int epi, const int8_t* q8_in, const in
   const int width = epi == kSiluPair ? rows / 2 : rows;
   if (m > 1 && out_stride < width) return hipErrorInvalidValue;
   GemmArgs a{epi, q8_in, xsum_in, scale_in, packed, scales, bias, output, rows, n, row_bytes, groups, out_stride, m};
+  if (work != nullptr && aligned16(work)) {
+    const size_t need = gemm_scaled_work(m, rows, n);
+    if (need > 0 && work_bytes >= (long long)need) return launch_gemm_scaled(stream, a, work);
+  }
   return launch_gemm(stream, a);
 }
 
@@ -416,9 +421,33 @@ hipError_t gemm_tile_silu_pair_wide(hipStream_t stream, IVONAR_GEMM_ARGS) {
   return GEMM_PASS_ENTRY(kSiluPair);
 }
 
-hipError_t ivonar_linear(hipStream_t stream, const void* input, int dtype, int m, void* work, const uint8_t* packed,
-                         const uint16_t* scales, const float* bias, float* output, int rows, int n, int row_bytes,
-                         int groups) {
+long long ivonar_gemm_work(int m, int rows, int n) {
+  return m <= 0 || rows <= 0 || n <= 0 ? 0 : (long long)gemm_scaled_work(m, rows, n);
+}
+
+hipError_t ivonar_gemm(hipStream_t stream, int epilogue, const int8_t* q8_in, const int32_t* xsum_in,
+                       const float* scale_in, const uint8_t* packed, const uint16_t* scales, const float* bias,
+                       float* output, int rows, int n, int row_bytes, int groups, int out_stride, int m, void* work,
+                       long long work_bytes) {
+  if (epilogue < kStore || epilogue > kSiluPair) return hipErrorInvalidValue;
+  return gemm_entry(stream, epilogue, q8_in, xsum_in, scale_in, packed, scales, bias, output, rows, n, row_bytes,
+                    groups, out_stride, m, work, work_bytes);
+}
+
+// Bytes of the quantized rows in ivonar_linear's workspace, rounded up to 16.
+static long long linear_rows_bytes(int m, int n) {
+  const long long chunks = ceil_div(n, kChunk);
+  return ((long long)m * (chunks * (kChunk + 4) + 4) + 15) & ~15LL;
+}
+
+long long ivonar_linear_work(int dtype, int m, int rows, int n) {
+  if (m <= 0 || rows <= 0 || n <= 0 || (m == 1 && dtype == kFloat32)) return 0;
+  return linear_rows_bytes(m, n) + (long long)gemm_scaled_work(m, rows, n);
+}
+
+hipError_t ivonar_linear(hipStream_t stream, const void* input, int dtype, int m, void* work, long long work_bytes,
+                         const uint8_t* packed, const uint16_t* scales, const float* bias, float* output, int rows,
+                         int n, int row_bytes, int groups) {
   const float* x = static_cast<const float*>(input);
   if (m == 1 && dtype == kFloat32)
     return gemv_entry(stream, kPlain, kStore, false, x, nullptr, nullptr, nullptr, nullptr, packed, scales, bias,
@@ -426,7 +455,8 @@ hipError_t ivonar_linear(hipStream_t stream, const void* input, int dtype, int m
   // Everything the second launch would refuse is refused before the first one goes out.
   hipError_t status = check_matrix(packed, scales, rows, n, row_bytes, groups);
   if (status != hipSuccess) return status;
-  if (dtype < kFloat32 || dtype > kBfloat16 || m < 0 || work == nullptr || output == nullptr)
+  if (dtype < kFloat32 || dtype > kBfloat16 || m < 0 || work == nullptr || output == nullptr ||
+      work_bytes < linear_rows_bytes(m, n))
     return hipErrorInvalidValue;
   const size_t chunks = (size_t)ceil_div(n, kChunk);
   int8_t* q8 = static_cast<int8_t*>(work);
@@ -437,8 +467,9 @@ hipError_t ivonar_linear(hipStream_t stream, const void* input, int dtype, int m
   if (m == 1)
     return gemv_entry(stream, kPlain, kStore, true, nullptr, nullptr, q8, xsum, scale, packed, scales, bias, output,
                       rows, n, row_bytes, groups, 1, 0.0f);
+  const long long used = linear_rows_bytes(m, n);
   return gemm_entry(stream, kStore, q8, xsum, scale, packed, scales, bias, output, rows, n, row_bytes, groups, rows,
-                    m);
+                    m, q8 + used, work_bytes - used);
 }
 int ivonar_linear_half(int n, const void* input) { return n > 0 && quantize_half_applies(n, input) ? 1 : 0; }
 

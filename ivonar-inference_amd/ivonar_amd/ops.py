@@ -33,7 +33,7 @@ _GEMV_NAMES = {
     ("attn", "residual"): "gemv_attn_residual",
 }
 _LINEAR_DTYPES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
-_GEMM_NAMES = {"store": "gemm_tile_store", "residual": "gemm_tile_residual", "silu_pair": "gemm_tile_silu_pair"}
+_GEMM_EPILOGUES = {"store": 0, "residual": 1, "silu_pair": 2}
 
 
 def _require_device(*tensors: Tensor | None) -> torch.device:
@@ -142,10 +142,12 @@ def gemm(
             raise KernelError("a residual GEMM needs the output tensor it adds into")
         out = torch.empty((rows, width), dtype=torch.float32, device=device)
     stride = int(out_stride if out_stride is not None else (out.stride(0) if out.ndim == 2 else width))
-    name = _GEMM_NAMES[epilogue]
-    _call(name, device, q8.data_ptr(), xsum.data_ptr(), scale.data_ptr(), matrix.packed.data_ptr(),
+    code = _GEMM_EPILOGUES[epilogue]
+    need = library().ivonar_gemm_work(rows, matrix.rows, matrix.in_features) if rows >= 128 else 0
+    work = torch.empty(need, dtype=torch.uint8, device=device) if need else None
+    _call("ivonar_gemm", device, code, q8.data_ptr(), xsum.data_ptr(), scale.data_ptr(), matrix.packed.data_ptr(),
           matrix.scales.data_ptr(), _address(matrix.bias), out.data_ptr(), matrix.rows, matrix.in_features,
-          matrix.row_bytes, matrix.groups, matrix.lanes, stride, rows)
+          matrix.row_bytes, matrix.groups, stride, rows, _address(work), need)
     return out
 
 
@@ -204,11 +206,10 @@ def ternary_linear(x: Tensor, matrix: Matrix) -> Tensor:
         rows, dtype = rows.float(), 0
     m = rows.numel() // width
     out = torch.empty((*lead, matrix.rows), dtype=torch.float32, device=device)
-    work = None
-    if m != 1 or dtype != 0:
-        # q8 rows, chunk sums and token scales of the call
-        work = torch.empty(m * (-(-width // CHUNK) * (CHUNK + 4) + 4), dtype=torch.uint8, device=device)
-    _call("ivonar_linear", device, rows.data_ptr(), dtype, m, _address(work), matrix.packed.data_ptr(),
+    # q8 rows, chunk sums and token scales of the call, and what its GEMM needs
+    need = library().ivonar_linear_work(dtype, m, matrix.rows, width)
+    work = torch.empty(need, dtype=torch.uint8, device=device) if need else None
+    _call("ivonar_linear", device, rows.data_ptr(), dtype, m, _address(work), need, matrix.packed.data_ptr(),
           matrix.scales.data_ptr(), _address(matrix.bias), out.data_ptr(), matrix.rows, width, matrix.row_bytes,
           matrix.groups)
     return out

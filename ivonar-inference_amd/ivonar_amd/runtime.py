@@ -26,7 +26,7 @@ from __future__ import annotations
 import ctypes
 import threading
 from collections.abc import Iterable, Mapping
-from ctypes import c_float, c_int, c_void_p
+from ctypes import c_float, c_int, c_longlong, c_void_p
 from pathlib import Path
 
 import torch
@@ -39,7 +39,7 @@ class KernelError(RuntimeError):
     pass
 
 
-_P, _I, _F = c_void_p, c_int, c_float
+_P, _I, _F, _L = c_void_p, c_int, c_float, c_longlong
 _GEMV = [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P, _I]
 _QUANT = [_P, _P, _I, _F, _I, _P, _P, _P]
 _QUANT_TILE = [_P, _I, _P, _I, _F, _I, _P, _P, _P]
@@ -62,7 +62,8 @@ SIGNATURES: dict[str, list] = {
         "gemm_tile_store", "gemm_tile_residual", "gemm_tile_silu_pair", "gemm_tile_store_wide",
         "gemm_tile_residual_wide", "gemm_tile_silu_pair_wide",
     )},
-    "ivonar_linear": [_P, _I, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I],
+    "ivonar_gemm": [_I, *_GEMM[:11], *_GEMM[12:], _P, _L],
+    "ivonar_linear": [_P, _I, _I, _P, _L, _P, _P, _P, _P, _I, _I, _I, _I],
     "embed_token": [_P, _P, _P, _P, _I, _I, _I],
     "embed_tile": [_P, _P, _P, _P, _I, _I, _I, _I],
     "gather_token": [_P, _P, _I, _P],
@@ -109,6 +110,10 @@ def library() -> ctypes.CDLL:
             lib.ivonar_gemm_plan.restype = c_int
             lib.ivonar_stream_read_sink_words.argtypes = []
             lib.ivonar_stream_read_sink_words.restype = c_int
+            lib.ivonar_gemm_work.argtypes = [c_int, c_int, c_int]
+            lib.ivonar_gemm_work.restype = c_longlong
+            lib.ivonar_linear_work.argtypes = [c_int, c_int, c_int, c_int]
+            lib.ivonar_linear_work.restype = c_longlong
             lib.ivonar_linear_half.argtypes = [c_int, c_void_p]
             lib.ivonar_linear_half.restype = c_int
             lib.ivonar_token_finish_limit.argtypes = [c_int]

@@ -64,5 +64,5 @@ def test_linear_refuses_what_it_cannot_run(cuda):
         ops.ternary_linear(torch.zeros(2, 256), matrix)
     x, out = torch.zeros(2, 256, device=cuda), torch.zeros(2, 64, device=cuda)
     tail = (matrix.packed.data_ptr(), matrix.scales.data_ptr(), None, out.data_ptr(), 64, 256, matrix.row_bytes, 2)
-    for dtype, work in ((3, x.data_ptr()), (0, None)):  # an unknown type, no workspace
-        assert runtime.library().ivonar_linear(0, x.data_ptr(), dtype, 2, work, *tail) != 0
+    for dtype, work, size in ((3, x.data_ptr(), 2048), (0, None, 2048), (0, x.data_ptr(), 16)):  # type, no or little work
+        assert runtime.library().ivonar_linear(0, x.data_ptr(), dtype, 2, work, size, *tail) != 0
