@@ -63,12 +63,13 @@ __device__ __forceinline__ float4 load4(const In* row, int i) {
 // exp(x): Cody-Waite reduction x = n*ln2 + r, degree-7 Taylor polynomial of
 // e^r in Horner form, scaling by 2^n in two exact steps.  Every operation is
 // an explicit IEEE fp32 op, so the CPU oracle reproduces it bit for bit.
+// Straight-line: the argument is clamped to where the steps are defined and
+// the special values are selected at the end, so that the outputs a lane
+// finishes together overlap (a branch on each kept them apart).
 __device__ __forceinline__ float ivo_expf(float x) {
-  if (x != x) return x;
-  if (x > 88.72283935546875f) return __builtin_inff();
-  if (x < -103.97208404541015625f) return 0.0f;
-  const float n = __builtin_rintf(x * 1.44269502162933349609375f);
-  float r = __builtin_fmaf(n, -0.693145751953125f, x);
+  const float c = fminf(fmaxf(x, -104.0f), 89.0f);  // NaN: -104
+  const float n = __builtin_rintf(c * 1.44269502162933349609375f);
+  float r = __builtin_fmaf(n, -0.693145751953125f, c);
   r = __builtin_fmaf(n, -1.428606765330187045e-06f, r);
   float p = 1.9841270113829523e-04f;
   p = __builtin_fmaf(p, r, 1.3888889225199819e-03f);
@@ -82,7 +83,10 @@ __device__ __forceinline__ float ivo_expf(float x) {
   const int n1 = ni / 2, n2 = ni - n1;
   const float s1 = __int_as_float((n1 + 127) << 23);
   const float s2 = __int_as_float((n2 + 127) << 23);
-  return (p * s1) * s2;
+  float y = (p * s1) * s2;
+  y = x > 88.72283935546875f ? __builtin_inff() : y;
+  y = x < -103.97208404541015625f ? 0.0f : y;
+  return x != x ? x : y;
 }
 
 __device__ __forceinline__ float ivo_silu(float x) { return x / (1.0f + ivo_expf(-x)); }
