@@ -31,19 +31,20 @@
 // bounded the kernel (K=4096 -> N=14336 at M=2048: 172 us against 138 on the
 // laid-out weights, two stages).
 //
-// gemm_scaled_kernel: a block of four waves owns 64 tokens x 384 rows, a wave
-// 64 tokens x 96 rows as 2 x 3 tiles of 32 x 32.  Three stages in LDS (two
-// blocks, 154 KB, on a CU), filled by direct buffer-to-LDS loads with two
+// gemm_scaled_kernel: a block of four waves owns 64 tokens x 128 NT rows, a wave
+// 64 tokens x 32 NT rows as 2 x NT tiles of 32 x 32 (NT = 1, 2 or 3).  Three
+// stages in LDS (two blocks, 154 KB with NT = 3, on a CU), filled by direct buffer-to-LDS loads with two
 // groups in flight, one barrier per group.  Per tile and group four MFMAs (two
 // halves of the 128 inputs, high and low part) with the previous tile's 16
 // fmaf between them.
 // Measured (one MI355X, graph replays, the lay-out's 10 us included): K=4096 ->
-// N=14336 at M=2048 158 -> 136 us (1.77 POPS), its silu-pair form 165 -> 149;
-// K=4096 -> N=22016 at M=777 115 -> 87 us.  What bounds it: the SIMD's issue
-// port.  An MFMA holds it for about 20 of its 32 cycles and each of the 5.5
-// VALU instructions per MFMA (4 of fold, 1.5 of expansion) for 4; without its
-// loads the kernel still takes 92% of the time, without the copies of operands
-// and per-group addresses that an earlier form had it gained 8%.
+// N=14336 at M=2048 154 -> 133 us (1.8 POPS), its silu-pair form 161 -> 144;
+// K=4096 -> N=22016 at M=777 113 -> 88; K=11008 -> N=4096 at M=777 75 -> 58.
+// What bounds it: the SIMD's issue port.  An MFMA holds it for about 20 of its
+// 32 cycles and each of the 5.5 VALU instructions per MFMA (4 of fold, 1.5 of
+// expansion) for 4; without its loads the kernel still takes 92% of the time,
+// without the copies of operands and per-group addresses that an earlier form
+// had it gained 8%.
 #include <type_traits>
 
 #include "buffer_ops.hpp"
@@ -58,9 +59,7 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 
 constexpr int kSplitGroupBytes = 192;  // FP6 high and low parts of one token's group
 constexpr int kScaledTokens = 64;
-constexpr int kRowTiles = 3;                       // 32-row tiles per wave
-constexpr int kWaveRows = 32 * kRowTiles;
-constexpr int kScaledRows = 4 * kWaveRows;
+constexpr int block_rows(int row_tiles) { return 128 * row_tiles; }  // four waves of 32-row tiles
 
 // Rows of the laid-out weights and scales: whole 16-byte pieces of scales.
 __host__ __device__ constexpr int row_pitch(int rows) { return (rows + 7) & ~7; }
@@ -208,22 +207,25 @@ __device__ __forceinline__ int inverse_bits(unsigned w, unsigned mask) {
   return d;
 }
 
+template <int NT>
 struct ScaledStage {
+  static constexpr int kRows = block_rows(NT);
   static constexpr int kTail = kScaledTokens * 128;            // after 8 head pieces of 16 bytes per token
   static constexpr int kWeights = kTail + kScaledTokens * 64;  // after 4 tail pieces per token
-  static constexpr int kScales = kWeights + kScaledRows * 32;  // after 2 pieces of weights per row
+  static constexpr int kScales = kWeights + kRows * 32;        // after 2 pieces of weights per row
   static constexpr int kBytes = kScales + 1024;                // fp16 per row
-  static_assert(kScaledRows * 2 <= 1024, "one wave instruction of scales");
+  static_assert(kRows * 2 <= 1024, "one wave instruction of scales");
 };
 
-template <int EPI>
+template <int EPI, int NT>
 __global__ __launch_bounds__(256, 2) void gemm_scaled_kernel(const unsigned char* __restrict__ rows6,
                                                              const uint4* __restrict__ weights_t,
                                                              const uint16_t* __restrict__ scales_t,
                                                              const float* __restrict__ scale_in,
                                                              const float* __restrict__ bias,
                                                              float* __restrict__ output, GemmArgs a, int nx, int ny) {
-  using S = ScaledStage;
+  using S = ScaledStage<NT>;
+  constexpr int kScaledRows = S::kRows, kWaveRows = 32 * NT;
   __shared__ __align__(16) unsigned char stages[3][S::kBytes];
   __shared__ __align__(16) float token_scales[kScaledTokens];
   const int tid = threadIdx.x;
@@ -243,23 +245,23 @@ __global__ __launch_bounds__(256, 2) void gemm_scaled_kernel(const unsigned char
 
   // Direct-to-LDS loads of a thread per group: two head pieces (slot
   // s = j*256 + tid: token s >> 3, piece (s & 7) ^ a_swizzle), one tail piece
-  // (token tid >> 2, piece (tid & 3) ^ (token >> 2 & 3)) and three pieces of
-  // weights (slot s = j*256 + tid of [half][384 rows]); wave 0 also loads the
+  // (token tid >> 2, piece (tid & 3) ^ (token >> 2 & 3)) and NT pieces of
+  // weights (slot s = j*256 + tid of [half][rows]); wave 0 also loads the
   // scales.  Tokens past m and rows past the pitch have a vector offset past
   // the buffer and read zeros (the scalar offset only moves by whole groups).
   constexpr int kPast = 0x7FFFFFF0;
   const int token_bytes = groups * kSplitGroupBytes;
   const int head_off = (token0 + (tid >> 3)) * token_bytes + ((tid & 7) ^ a_swizzle(tid >> 3)) * 16;
   const int tail_off = (token0 + (tid >> 2)) * token_bytes + 128 + ((tid & 3) ^ ((tid >> 4) & 3)) * 16;
-  int w_off[3];
+  int w_off[NT];
 #pragma unroll
-  for (int j = 0; j < 3; ++j) {
+  for (int j = 0; j < NT; ++j) {
     const int s = j * 256 + tid, h = s >= kScaledRows, row = row0 + s - h * kScaledRows;
     w_off[j] = row < pitch ? (h * pitch + row) * 16 : kPast;
   }
-  static_assert(kScaledRows * 2 == 3 * 256, "three pieces of weights per thread");
+  static_assert(kScaledRows * 2 == NT * 256, "whole pieces of weights per thread");
   const int s_off = row0 + lane * 8 < pitch ? row0 * 2 + lane * 16 : kPast;
-  constexpr int kLoads = 6;  // per group, and one more in wave 0
+  constexpr int kLoads = 3 + NT;  // per group, and one more in wave 0
   const unsigned lds_base = __builtin_amdgcn_readfirstlane(lds_address(&stages[0][0]) + wave * 1024);
   auto load = [&](int g, int stage) {
     const unsigned base = lds_base + stage * S::kBytes;
@@ -269,15 +271,15 @@ __global__ __launch_bounds__(256, 2) void gemm_scaled_kernel(const unsigned char
     for (int j = 0; j < 2; ++j) dma16(q_buf, base + j * 4096, head_off + j * 32 * token_bytes, g * kSplitGroupBytes);
     dma16(q_buf, base + S::kTail, tail_off, g * kSplitGroupBytes);
 #pragma unroll
-    for (int j = 0; j < 3; ++j) dma16(w_buf, base + S::kWeights + j * 4096, w_off[j], g * pitch * 32);
+    for (int j = 0; j < NT; ++j) dma16(w_buf, base + S::kWeights + j * 4096, w_off[j], g * pitch * 32);
     if (wave == 0) dma16(s_buf, base + S::kScales, s_off, scale_group * pitch * 2);
   };
 
-  v16f acc[2][kRowTiles];
+  v16f acc[2][NT];
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < kRowTiles; ++nt) acc[mt][nt] = v16f{};
+    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = v16f{};
   // The previous tile's P and scale, folded while the next tile's MFMAs run
   // (zero before the first: a fold of zeros leaves acc at +0).
   v16f prev{};
@@ -336,17 +338,17 @@ __global__ __launch_bounds__(256, 2) void gemm_scaled_kernel(const unsigned char
                  inverse_bits(w1 << 2, 0xCCCCCCCCu), inverse_bits(w1, 0xCCCCCCCCu), 0, 0, 0, 0};
     };
 #pragma unroll
-    for (int nt = 0; nt < kRowTiles; ++nt) {
+    for (int nt = 0; nt < NT; ++nt) {
       expand(0);
       expand(1);
       const float tile_sc = sc;
-      if (nt + 1 < kRowTiles) {
+      if (nt + 1 < NT) {
         raw = *reinterpret_cast<const uint4*>(w_read + kOffset + (nt + 1) * 32 * 16);
         sc = h2f(*reinterpret_cast<const uint16_t*>(s_read + kOffset + (nt + 1) * 64));
       }
 #pragma unroll
       for (int mt = 0; mt < 2; ++mt) {
-        const int fold_mt = mt ^ 1, fold_nt = mt ? nt : (nt + kRowTiles - 1) % kRowTiles;
+        const int fold_mt = mt ^ 1, fold_nt = mt ? nt : (nt + NT - 1) % NT;
         v16f p{};
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -370,7 +372,7 @@ __global__ __launch_bounds__(256, 2) void gemm_scaled_kernel(const unsigned char
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < kRowTiles; ++nt) asm volatile("" : "+v"(acc[mt][nt]));
+      for (int nt = 0; nt < NT; ++nt) asm volatile("" : "+v"(acc[mt][nt]));
   };
   // Three steps per round, so that every stage is a constant; steps past the
   // last group run it again with the zero scales laid out behind the last
@@ -384,7 +386,7 @@ __global__ __launch_bounds__(256, 2) void gemm_scaled_kernel(const unsigned char
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
   for (int i = 0; i < 16; ++i)
-    acc[1][kRowTiles - 1][i] = __builtin_fmaf(prev[i], prev_sc, acc[1][kRowTiles - 1][i]);
+    acc[1][NT - 1][i] = __builtin_fmaf(prev[i], prev_sc, acc[1][NT - 1][i]);
 
   // Epilogue.  A lane holds row c of a tile for the 16 tokens
   // 8*(i >> 2) + 4*half + (i & 3): 32 lanes write 128 contiguous bytes of an
@@ -398,9 +400,9 @@ __global__ __launch_bounds__(256, 2) void gemm_scaled_kernel(const unsigned char
   const bool has_bias = bias != nullptr;
   const int stride4 = a.out_stride * 4;
   constexpr int kStream = 2;  // non-temporal: the output is written once
-  float bv[kRowTiles];
+  float bv[NT];
 #pragma unroll
-  for (int nt = 0; nt < kRowTiles; ++nt)
+  for (int nt = 0; nt < NT; ++nt)
     bv[nt] = has_bias ? bias[min(row0 + wave * kWaveRows + nt * 32 + c, a.rows - 1)] : 0.0f;
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt) {
@@ -413,7 +415,7 @@ __global__ __launch_bounds__(256, 2) void gemm_scaled_kernel(const unsigned char
     }
     const int t_off = (mt * 32 + 4 * half) * stride4;
 #pragma unroll
-    for (int nt = 0; nt < kRowTiles; ++nt) {
+    for (int nt = 0; nt < NT; ++nt) {
       const int row = row0 + wave * kWaveRows + nt * 32 + c;
       const bool live = row < a.rows;
       const int off = live ? t_off + (EPI == kSiluPair ? row >> 1 : row) * 4 : kPast;
@@ -469,12 +471,21 @@ ScaledWork scaled_work(int m, int rows, int n) {
   return w;
 }
 
-template <int EPI>
-hipError_t launch_scaled_epi(hipStream_t stream, const GemmArgs& a, const LayOut& l) {
-  const int nx = ceil_div(a.rows, kScaledRows), ny = ceil_div(a.m, kScaledTokens);
-  hipLaunchKernelGGL(gemm_scaled_kernel<EPI>, dim3(nx * ny), dim3(256), 0, stream, l.rows6, l.weights, l.scales_t,
+template <int EPI, int NT>
+hipError_t launch_scaled_shape(hipStream_t stream, const GemmArgs& a, const LayOut& l) {
+  const int nx = ceil_div(a.rows, block_rows(NT)), ny = ceil_div(a.m, kScaledTokens);
+  hipLaunchKernelGGL((gemm_scaled_kernel<EPI, NT>), dim3(nx * ny), dim3(256), 0, stream, l.rows6, l.weights, l.scales_t,
                      a.scale_in, a.bias, a.output, a, nx, ny);
   return hipGetLastError();
+}
+
+template <int EPI>
+hipError_t launch_scaled_epi(hipStream_t stream, const GemmArgs& a, const LayOut& l, int row_tiles) {
+  switch (row_tiles) {
+    case 1: return launch_scaled_shape<EPI, 1>(stream, a, l);
+    case 2: return launch_scaled_shape<EPI, 2>(stream, a, l);
+    default: return launch_scaled_shape<EPI, 3>(stream, a, l);
+  }
 }
 
 }  // namespace
@@ -490,33 +501,61 @@ float round_time(long long tiles, int cus, float two, float one) {
 
 }  // namespace
 
-// Where it is used: prompts that gemm_wide_kernel's 128-token tiles would take
-// (2048 inputs and more), if the tiles of this kernel are expected to finish
-// first, the lay-out included.  Both kernels' steps take a constant time while
-// their blocks fill the CUs alike, so the expectation is a step time times the
-// rounds of blocks.  Fitted on (K -> N, M; 128-token int8 tiles against this
-// kernel with its lay-out, store): 4096 -> 14336, 2048: 158 against 136 us;
-// 4096 -> 22016, 777: 115 / 87; 4096 -> 12288, 777: 76 / 57; 8192 -> 8192, 2048:
-// 157 / 159 (one full round of 512 int8 blocks, 1.4 of these); 4096 -> 4096,
-// 2048: 47 / 56; 4096 -> 14336, 512: 46 / 54.
-size_t gemm_scaled_work(int m, int rows, int n) {
-  if (gemm_wide_tokens(m, rows, n) != 128) return 0;
+namespace {
+
+// Row tiles per wave (1, 2 or 3: blocks of 128, 256 or 384 rows), 0 where the
+// int8 kernel is expected to finish first: prompts that gemm_wide_kernel would
+// take with 2048 inputs and more.  The steps of either kernel take a constant
+// time while its blocks fill the CUs alike, so the expected time is a step time
+// (us, with two blocks and with one on a CU) times the rounds of blocks, and
+// for this kernel the lay-out (its bytes at 6 TB/s) and 10 us of launch,
+// prologue and epilogue.  Narrow blocks cost more per output and win where wide
+// ones leave CUs idle.  Fitted on these (K -> N, M: int8; 1, 2, 3 row tiles,
+// lay-out included, us):
+//   4096 -> 14336, 2048: 154; 150, 133, 133     4096 -> 22016, 777: 113; 100, 97, 88
+//   4096 -> 12288, 777: 75; 61, 64, 58          11008 -> 4096, 777: 75; 58, 65, 83
+//   8192 -> 8192, 2048: 157; 169, 153, 159      4096 -> 4096, 777: 33; 33, 36, 42
+//   4096 -> 4096, 2048: 47; 54, 47, 55          4096 -> 14336, 512: 48; 53, 45, 55
+//   2048 -> 6144, 1024: 27; 28, 28, 30          4096 -> 12288, 300: 30; 31, 34, 39
+// Below 2048 inputs the int8 kernel won (1024 -> 4096, 2048: 17; 22, 21, 23).
+int scaled_row_tiles(int m, int rows, int n) {
   const int groups = ceil_div(n, kGroup), cus = device_cus();
+  const int int8_tokens = gemm_wide_tokens(m, rows, n);
   const long long limit = 0x7FFFFFF0LL;  // 32-bit buffer offsets, a tile of slack
-  if ((m + (long long)kScaledTokens) * groups * kSplitGroupBytes >= limit ||
-      (rows + (long long)kScaledRows) * groups * 32 >= limit)
+  if (int8_tokens < 64 || groups < 16 || (m + (long long)kScaledTokens) * groups * kSplitGroupBytes >= limit ||
+      (rows + (long long)block_rows(3)) * groups * 32 >= limit)
     return 0;
-  const long long int8_tiles = (long long)ceil_div(rows, 256) * ceil_div(m, 128);
-  const long long tiles = (long long)ceil_div(rows, kScaledRows) * ceil_div(m, kScaledTokens);
-  const float lay_out = 7.0f + ((float)m * 320.0f + (float)rows * 68.0f) * (float)groups / 6.0e6f;
-  const float int8_time = (float)groups * round_time(int8_tiles, cus, 2.45f, 1.45f);
-  const float time = (float)padded_groups(groups) * round_time(tiles, cus, 1.24f, 0.95f) + lay_out;
-  return time * 1.03f < int8_time ? scaled_work(m, rows, n).bytes : 0;
+  const long long int8_tiles = (long long)ceil_div(rows, 256) * ceil_div(m, int8_tokens);
+  float best = (float)groups * (int8_tokens == 128 ? round_time(int8_tiles, cus, 2.45f, 1.45f)
+                                                   : round_time(int8_tiles, cus, 1.4f, 0.85f)) +
+               (int8_tokens == 128 ? 0.0f : 5.0f);
+  best *= 0.97f;  // no change for less than the fit's error
+  const float lay_out = 10.0f + ((float)m * 320.0f + (float)rows * 68.0f) * (float)groups / 6.0e6f;
+  constexpr float kStep[3][2] = {{0.56f, 0.33f}, {0.97f, 0.55f}, {1.25f, 0.82f}};
+  int choice = 0;
+  for (int tiles = 1; tiles <= 3; ++tiles) {
+    const long long blocks = (long long)ceil_div(rows, block_rows(tiles)) * ceil_div(m, kScaledTokens);
+    const float time =
+        (float)padded_groups(groups) * round_time(blocks, cus, kStep[tiles - 1][0], kStep[tiles - 1][1]) + lay_out;
+    if (time < best) {
+      best = time;
+      choice = tiles;
+    }
+  }
+  return choice;
+}
+
+}  // namespace
+
+size_t gemm_scaled_work(int m, int rows, int n) {
+  return scaled_row_tiles(m, rows, n) == 0 ? 0 : scaled_work(m, rows, n).bytes;
 }
 
 hipError_t launch_gemm_scaled(hipStream_t stream, const GemmArgs& a, void* work) {
   // 32-bit buffer offsets into a block's output rows.
   if ((2 * kScaledTokens + 1LL) * a.out_stride * 4 + 4LL * a.rows >= 0x7FFFFFF0LL) return launch_gemm(stream, a);
+  const int wave_tiles = scaled_row_tiles(a.m, a.rows, a.n);
+  if (wave_tiles == 0) return launch_gemm(stream, a);
   const ScaledWork w = scaled_work(a.m, a.rows, a.n);
   unsigned char* base = static_cast<unsigned char*>(work);
   LayOut l{};
@@ -542,9 +581,9 @@ hipError_t launch_gemm_scaled(hipStream_t stream, const GemmArgs& a, void* work)
   const hipError_t status = hipGetLastError();
   if (status != hipSuccess) return status;
   switch (a.epi) {
-    case kStore: return launch_scaled_epi<kStore>(stream, a, l);
-    case kResidual: return launch_scaled_epi<kResidual>(stream, a, l);
-    case kSiluPair: return launch_scaled_epi<kSiluPair>(stream, a, l);
+    case kStore: return launch_scaled_epi<kStore>(stream, a, l, wave_tiles);
+    case kResidual: return launch_scaled_epi<kResidual>(stream, a, l, wave_tiles);
+    case kSiluPair: return launch_scaled_epi<kSiluPair>(stream, a, l, wave_tiles);
     default: return hipErrorInvalidValue;
   }
 }

@@ -1,5 +1,5 @@
 """The block-scaled FP6 x FP4 token GEMM: the bits of the int8 kernels (themselves checked against the oracle) on
-every output, at the edges of its tiles (64 tokens, 384 rows, 8-row pitch), with group counts of every remainder
+every output, at the edges of its tiles (64 tokens, 128, 256 or 384 rows, 8-row pitch), with group counts of every remainder
 of its three-step rounds, an odd chunk count, all three epilogues, a bias and a padded output stride; and a sample of
 token rows against the oracle."""
 
@@ -16,8 +16,10 @@ pytestmark = pytest.mark.gpu
 NAMES = {"store": "gemm_tile_store", "residual": "gemm_tile_residual", "silu_pair": "gemm_tile_silu_pair"}
 
 
+# Row tiles per wave: three, and one and two where they fill the CUs better (11008 inputs to 4096 rows; 8192 to 8194).
 @pytest.mark.parametrize("m,k,rows", [(777, 4096, 12288), (705, 4224, 12290), (704, 4352, 12286), (640, 2112, 30002),
-                                      (2047, 2048, 14338)])
+                                      (2047, 2048, 14338), (777, 11008, 4096), (833, 11072, 4098), (2048, 8192, 8192),
+                                      (2001, 8320, 8194)])
 @pytest.mark.parametrize("epilogue", sorted(NAMES))
 def test_gemm_scaled_matches_the_int8_kernels(cuda, oracle, m, k, rows, epilogue):
     import torch
