@@ -475,7 +475,8 @@ def measure_mfma(calls: int = 16, cus: int = 256, xcds: int = 8) -> dict:
     rows = counter_pass(counters, "gemm-prefill", calls)
     if isinstance(rows, str):
         return {"error": rows}
-    kernels = ("gemm_kernel", "gemm_wide_kernel", "gemm_split_kernel", "skinny_kernel", "skinny_row_kernel")
+    kernels = ("gemm_kernel", "gemm_wide_kernel", "gemm_split_kernel", "gemm_scaled_kernel", "skinny_kernel",
+               "skinny_row_kernel")
     gemm = [row for row in rows if any(name in row["kernel"] for name in kernels) and all(c in row for c in counters)]
     cases = [(k, n, m) for k, n in PROBE_GEMM_SHAPES for m in PROBE_GEMM_M]
     if len(gemm) != len(cases) * calls:
@@ -494,7 +495,8 @@ def measure_mfma(calls: int = 16, cus: int = 256, xcds: int = 8) -> dict:
                                   "mfma_ops_counted": int(mean("SQ_INSTS_VALU_MFMA_MOPS_I8") * 512),
                                   "ops_algorithmic": 2 * m * n * k, "kernel": name}
     return {"by_case": table, "simds": 4 * cus,
-            "note": "GRBM_GUI_ACTIVE covers the whole dispatch under counter collection, launch and drain included"}
+            "note": "GRBM_GUI_ACTIVE covers the whole dispatch under counter collection, launch and drain included; "
+                    "gemm_scaled_kernel's MFMAs are FP6 x FP4 and not in the int8 count"}
 
 
 def m_sweep(device, stream) -> dict:
