@@ -10,7 +10,7 @@
 // gemm_wide_kernel.  v_mfma_scale_f32_32x32x64_f8f6f4 accumulates in fp32, so
 // P arrives as a float and only the fmaf is left, and it takes operands that
 // hold both factors exactly:
-//   * an int8 value q = s * (16 h + l), s its sign, h in 0..7, l in 0..15: the
+//   * an int8 value q = s * (16 h + l), s its sign, h in 0..8, l in 0..15: the
 //     FP6 (E2M3) numbers s*h/8 and s*l/8 (their codes are the integers
 //     themselves), weighted by the block scales 2^6 and 2^2;
 //   * a ternary weight as the FP4 (E2M1) number -2, 0 or +2: bit 3 (sign) is
@@ -74,8 +74,8 @@ __device__ __forceinline__ unsigned pack6(unsigned bytes) {
 }
 __device__ __forceinline__ void split6(unsigned q, unsigned& high, unsigned& low) {
   const unsigned sign = (q >> 7) & 0x01010101u;
-  const unsigned magnitude = (q ^ ((sign << 8) - sign)) + sign;  // per byte: |q| <= 127
-  high = pack6(((magnitude >> 4) & 0x07070707u) | (sign << 5));
+  const unsigned magnitude = (q ^ ((sign << 8) - sign)) + sign;  // per byte: |q| <= 128
+  high = pack6(((magnitude >> 4) & 0x0F0F0F0Fu) | (sign << 5));
   low = pack6((magnitude & 0x0F0F0F0Fu) | (sign << 5));
 }
 
