@@ -18,7 +18,7 @@
  *     least 16*ceil(n/64); byte b holds inputs 4b..4b+3, input 4b+k in bits
  *     2k..2k+1 as code = w + 1 (w in {-1,0,+1}).  16-byte aligned.
  *   - scales: fp16 bit patterns [rows, groups], groups >= ceil(n/128), one
- *     scale per 128 inputs.  bias: fp32 [rows] or NULL.
+ *     scale per 128 inputs, at any even address.  bias: fp32 [rows] or NULL.
  *   - q8/xsum/scale buffers hold quantized activations in this library's
  *     private layout; capacity per token row: ceil(n/64)*64 int8,
  *     ceil(n/64) int32 and one fp32 (the reference's q8/q8sum/q8scale sizes).

@@ -281,9 +281,12 @@ __global__ __launch_bounds__(64 * S) void skinny_row_kernel(const int8_t* __rest
   constexpr int kPast = 0x7FFFFFF0;
   const v4u q8_buf = wide_buffer(q8, (long long)m * q8_stride);
   const v4u w_buf = wide_buffer(packed, (long long)a.rows * a.row_bytes);
-  // The scales are fetched as dwords and the range check drops a dword that ends past the size: an odd
-  // count of halfwords is rounded up, so that the last scale's dword counts (it shares its dword's page).
-  const v4u s_buf = wide_buffer(scales, ((long long)a.rows * a.groups * 2 + 3) & ~3LL);
+  // The scales are fetched as dwords, so the buffer runs over whole dwords of memory: from the one that
+  // holds the first scale (a caller's array may start in its middle) to the one that holds the last (the
+  // range check drops a dword that ends past the size).  Neither end leaves the scales' own dwords.
+  const int scale_start = (int)(reinterpret_cast<uintptr_t>(scales) & 2);
+  const v4u s_buf = wide_buffer(reinterpret_cast<const unsigned char*>(scales) - scale_start,
+                                ((long long)a.rows * a.groups * 2 + scale_start + 3) & ~3LL);
 
   // What the epilogue reads from global memory (token scales, biases, residual
   // bases of this thread's outputs) goes out first: older than every
@@ -305,7 +308,7 @@ __global__ __launch_bounds__(64 * S) void skinny_row_kernel(const int8_t* __rest
   }
 
   // Scales: lane l < 16R fetches row row0 + l from group g0 on, 32 bytes from the dword below.
-  const int scale_byte = ((row0 + lane) * a.groups + g0) * 2;
+  const int scale_byte = ((row0 + lane) * a.groups + g0) * 2 + scale_start;
   const int scale_shift = scale_byte & 3;
   const bool scale_lane = lane < 16 * R && row0 + lane < a.rows;
   dma16(s_buf, s_lds, scale_lane ? scale_byte - scale_shift : kPast, 0);

@@ -147,8 +147,8 @@ __global__ __launch_bounds__(64 * kMaxWaves) void token_gemv_kernel(const int8_t
   const uint8_t* wrow = packed + (size_t)row * sh.row_bytes + (size_t)(g_first / 2 + span0) * kSpanBytes + kb * 16;
   const uint16_t* srow = scales + (size_t)row * sh.groups + g_first + span0 * 2;
   unsigned sc[PART];  // the two fp16 group scales of each span
-  if ((sh.groups & 1) == 0) {
-    // Even scale rows: every span's scale pair sits at a multiple of 4 bytes.
+  if ((sh.groups & 1) == 0 && (reinterpret_cast<uintptr_t>(scales) & 2) == 0) {
+    // Even scale rows from a 4-byte boundary: every span's scale pair sits at a multiple of 4 bytes.
 #pragma unroll
     for (int i = 0; i < PART; i += 2) {
       if (i + 1 < PART) {
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(64 * kMaxWaves) void token_gemv_kernel(const int8_t
       }
     }
   } else {
-    // Odd scale rows (padded past K / 128 groups): 2-byte aligned, one fp16 per load.
+    // Odd scale rows (padded past K / 128 groups) or an array off a 4-byte boundary: one fp16 per load.
 #pragma unroll
     for (int i = 0; i < PART; ++i) sc[i] = (unsigned)srow[2 * i] | ((unsigned)srow[2 * i + 1] << 16);
   }
