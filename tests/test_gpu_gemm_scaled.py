@@ -77,6 +77,32 @@ def test_small_workspace_runs_the_int8_kernel(cuda):
     assert lib.ivonar_gemm(0, 3, *([None] * 7), rows, k, matrix.row_bytes, matrix.groups, rows, m, None, 0) != 0
 
 
+def test_no_memory_for_the_workspace_runs_the_int8_kernel(cuda, monkeypatch):
+    """The allocation of the block-scaled kernel's workspace fails (forced here): the call runs without it."""
+    import torch
+    from ivonar_amd import ops
+
+    m, k, rows = 777, 4096, 12288
+    rng = np.random.default_rng(4)
+    _, packed, scale_bits, _ = make_layer(rng, rows, k)
+    matrix = device_matrix(packed, scale_bits, k, device=cuda)
+    x = torch.randn(m, k, device=cuda)
+    expected = ops.ternary_linear(x, matrix)
+    buffers = ops.quantize_rows(x)
+    refused, real = [], torch.empty
+
+    def empty(*args, **kwargs):
+        if kwargs.get("dtype") == torch.uint8 and args[0] > m * k * 2:
+            refused.append(args[0])
+            raise torch.OutOfMemoryError("forced")
+        return real(*args, **kwargs)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    assert torch.equal(ops.ternary_linear(x, matrix), expected)
+    assert torch.equal(ops.gemm(matrix, *buffers), expected)
+    assert len(refused) == 2
+
+
 def test_graph_replays_with_the_workspace(cuda):
     import torch
     from ivonar_amd import ops
