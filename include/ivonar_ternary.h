@@ -191,8 +191,10 @@ hipError_t gemm_tile_silu_pair_wide(hipStream_t stream, IVONAR_GEMM_ARGS);
  * ivonar_gemm_work(m, rows, n), and that not 0, the long-prompt kernel on the
  * block-scaled MFMA runs (the same results bit for bit); else gemm_tile_*.
  * The workspace is written before it is read and free again once the call has
- * run. */
+ * run.  ivonar_gemm_row_tiles: the 32-row tiles per wave (1, 2 or 3) that kernel
+ * takes, 0 where the int8 kernels run.  Both host only. */
 long long ivonar_gemm_work(int m, int rows, int n);
+int ivonar_gemm_row_tiles(int m, int rows, int n);
 hipError_t ivonar_gemm(hipStream_t stream, int epilogue, const int8_t* q8_in, const int32_t* xsum_in,
                        const float* scale_in, const uint8_t* packed, const uint16_t* scales, const float* bias,
                        float* output, int rows, int n, int row_bytes, int groups, int out_stride, int m, void* work,

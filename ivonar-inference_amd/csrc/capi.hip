@@ -425,6 +425,10 @@ long long ivonar_gemm_work(int m, int rows, int n) {
   return m <= 0 || rows <= 0 || n <= 0 ? 0 : (long long)gemm_scaled_work(m, rows, n);
 }
 
+int ivonar_gemm_row_tiles(int m, int rows, int n) {
+  return m <= 0 || rows <= 0 || n <= 0 ? 0 : gemm_scaled_row_tiles(m, rows, n);
+}
+
 hipError_t ivonar_gemm(hipStream_t stream, int epilogue, const int8_t* q8_in, const int32_t* xsum_in,
                        const float* scale_in, const uint8_t* packed, const uint16_t* scales, const float* bias,
                        float* output, int rows, int n, int row_bytes, int groups, int out_stride, int m, void* work,

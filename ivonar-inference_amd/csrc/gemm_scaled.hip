@@ -37,9 +37,9 @@
 // groups in flight, one barrier per group.  Per tile and group four MFMAs (two
 // halves of the 128 inputs, high and low part) with the previous tile's 16
 // fmaf between them.
-// Measured (one MI355X, graph replays, the lay-out's 10 us included): K=4096 ->
-// N=14336 at M=2048 154 -> 133 us (1.8 POPS), its silu-pair form 161 -> 144;
-// K=4096 -> N=22016 at M=777 113 -> 88; K=11008 -> N=4096 at M=777 75 -> 58.
+// Measured (one MI355X, graph replays, the lay-out's 10 us included, the int8
+// kernel before): K=4096 -> N=14336 at M=2048 168 -> 137 us (1.75 POPS); K=4096
+// -> N=22016 at M=777 123 -> 93; K=11008 -> N=4096 at M=777 72 -> 55.
 // What bounds it: the SIMD's issue port.  An MFMA holds it for about 20 of its
 // 32 cycles and each of the 5.5 VALU instructions per MFMA (4 of fold, 1.5 of
 // expansion) for 4; without its loads the kernel still takes 92% of the time,
@@ -488,55 +488,64 @@ hipError_t launch_scaled_epi(hipStream_t stream, const GemmArgs& a, const LayOut
   }
 }
 
-}  // namespace
+// Time (us) of one group step of a kernel whose blocks go two to a CU, by the blocks that are left: with one
+// block on one CU, one on every CU, two on one CU, two on every CU.
+struct StepTimes {
+  float one, all, second, both;
+};
 
-namespace {
-
-// Time of one group step over `tiles` blocks of which two share a CU, from the
-// times of a step with two blocks on every CU and with at most one.
-float round_time(long long tiles, int cus, float two, float one) {
-  const long long rest = tiles % (2 * cus);
-  return (float)(tiles / (2 * cus)) * two + (rest == 0 ? 0.0f : rest <= cus ? one : two);
+// Time of a group step over `blocks` blocks: whole rounds of two blocks per CU, then the rest.  A rest past
+// one block per CU makes a step: the CUs that hold two blocks take the pair's time, however few they are.
+float round_time(long long blocks, int cus, const StepTimes& t) {
+  const long long rest = blocks % (2 * cus);
+  const float whole = (float)(blocks / (2 * cus)) * t.both;
+  if (rest == 0) return whole;
+  if (rest <= cus) return whole + t.one + (t.all - t.one) * (float)rest / (float)cus;
+  return whole + t.second + (t.both - t.second) * (float)(rest - cus) / (float)cus;
 }
 
 }  // namespace
 
-namespace {
-
 // Row tiles per wave (1, 2 or 3: blocks of 128, 256 or 384 rows), 0 where the
 // int8 kernel is expected to finish first: prompts that gemm_wide_kernel would
-// take with 2048 inputs and more.  The steps of either kernel take a constant
-// time while its blocks fill the CUs alike, so the expected time is a step time
-// (us, with two blocks and with one on a CU) times the rounds of blocks, and
-// for this kernel the lay-out (its bytes at 6 TB/s) and 10 us of launch,
-// prologue and epilogue.  Narrow blocks cost more per output and win where wide
-// ones leave CUs idle.  Fitted on these (K -> N, M: int8; 1, 2, 3 row tiles,
-// lay-out included, us):
-//   4096 -> 14336, 2048: 154; 150, 133, 133     4096 -> 22016, 777: 113; 100, 97, 88
-//   4096 -> 12288, 777: 75; 61, 64, 58          11008 -> 4096, 777: 75; 58, 65, 83
-//   8192 -> 8192, 2048: 157; 169, 153, 159      4096 -> 4096, 777: 33; 33, 36, 42
-//   4096 -> 4096, 2048: 47; 54, 47, 55          4096 -> 14336, 512: 48; 53, 45, 55
-//   2048 -> 6144, 1024: 27; 28, 28, 30          4096 -> 12288, 300: 30; 31, 34, 39
-// Below 2048 inputs the int8 kernel won (1024 -> 4096, 2048: 17; 22, 21, 23).
-int scaled_row_tiles(int m, int rows, int n) {
+// take with 2048 inputs and more.  The expected time of either kernel is a
+// constant plus a group step's time over its blocks (round_time) times the
+// groups; for this kernel the constant is 11.8 us (launch, prologue, epilogue,
+// the lay-out's launch) and the lay-out's bytes at 10 TB/s.  Narrow blocks cost
+// more per output and win where wide ones leave CUs idle.  Fitted on 257 shapes
+// of 128..4096 tokens (graph replays, weights warm, one MI355X) with a mean error
+// of 4%.  On those the choice is on average 0.3% slower than the best, at worst
+// 14%, and at worst 1% slower than the int8 kernel; on 181 others of random sizes
+// 0.6%, 12% and 1.5%.  Some (us; int8, then 1, 2, 3 row tiles, lay-out included):
+//   4096 -> 14336, 2048: 168; 150, 137, 141     4096 -> 22016, 777: 123; 101, 101, 93
+//   4096 -> 12288, 777: 78; 61, 66, 59          11008 -> 4096, 777: 72; 55, 64, 80
+//   8192 -> 8192, 2048: 179; 171, 155, 167      4096 -> 4096, 777: 30; 30, 34, 40
+//   4096 -> 4096, 2048: 55; 57, 50, 60          4096 -> 14336, 514: 76; 53, 47, 56
+//   2048 -> 6144, 1024: 28; 29, 29, 30          4096 -> 12288, 300: 31; 31, 34, 40
+// (Charging a partly filled round the time of a full one, the rule took two row
+// tiles for 11008 -> 4096 and for 4096 -> 4096 at 777, 13% behind the int8 kernel
+// at worst.)
+// Below 2048 inputs the comparison is not made (1024 -> 4096, 2048: int8 17;
+// 22, 21, 23).
+int gemm_scaled_row_tiles(int m, int rows, int n) {
   const int groups = ceil_div(n, kGroup), cus = device_cus();
   const int int8_tokens = gemm_wide_tokens(m, rows, n);
   const long long limit = 0x7FFFFFF0LL;  // 32-bit buffer offsets, a tile of slack
   if (int8_tokens < 64 || groups < 16 || (m + (long long)kScaledTokens) * groups * kSplitGroupBytes >= limit ||
       (rows + (long long)block_rows(3)) * groups * 32 >= limit)
     return 0;
-  const long long int8_tiles = (long long)ceil_div(rows, 256) * ceil_div(m, int8_tokens);
-  float best = (float)groups * (int8_tokens == 128 ? round_time(int8_tiles, cus, 2.45f, 1.45f)
-                                                   : round_time(int8_tiles, cus, 1.4f, 0.85f)) +
-               (int8_tokens == 128 ? 0.0f : 5.0f);
-  best *= 0.97f;  // no change for less than the fit's error
-  const float lay_out = 10.0f + ((float)m * 320.0f + (float)rows * 68.0f) * (float)groups / 6.0e6f;
-  constexpr float kStep[3][2] = {{0.56f, 0.33f}, {0.97f, 0.55f}, {1.25f, 0.82f}};
+  const long long int8_blocks = (long long)ceil_div(rows, 256) * ceil_div(m, int8_tokens);
+  const float int8_time = int8_tokens == 128
+                              ? 7.9f + (float)groups * round_time(int8_blocks, cus, {0.885f, 1.36f, 2.13f, 2.6f})
+                              : 4.75f + (float)groups * round_time(int8_blocks, cus, {0.43f, 0.88f, 1.31f, 1.85f});
+  float best = 0.97f * int8_time;  // no change for less than the fit's error
+  const float lay_out = 11.8f + ((float)m * 320.0f + (float)rows * 68.0f) * (float)groups / 10.0e6f;
+  constexpr StepTimes kStep[3] = {
+      {0.124f, 0.277f, 0.396f, 0.586f}, {0.416f, 0.599f, 0.769f, 1.05f}, {0.568f, 0.889f, 1.2f, 1.51f}};
   int choice = 0;
   for (int tiles = 1; tiles <= 3; ++tiles) {
     const long long blocks = (long long)ceil_div(rows, block_rows(tiles)) * ceil_div(m, kScaledTokens);
-    const float time =
-        (float)padded_groups(groups) * round_time(blocks, cus, kStep[tiles - 1][0], kStep[tiles - 1][1]) + lay_out;
+    const float time = (float)padded_groups(groups) * round_time(blocks, cus, kStep[tiles - 1]) + lay_out;
     if (time < best) {
       best = time;
       choice = tiles;
@@ -545,16 +554,14 @@ int scaled_row_tiles(int m, int rows, int n) {
   return choice;
 }
 
-}  // namespace
-
 size_t gemm_scaled_work(int m, int rows, int n) {
-  return scaled_row_tiles(m, rows, n) == 0 ? 0 : scaled_work(m, rows, n).bytes;
+  return gemm_scaled_row_tiles(m, rows, n) == 0 ? 0 : scaled_work(m, rows, n).bytes;
 }
 
 hipError_t launch_gemm_scaled(hipStream_t stream, const GemmArgs& a, void* work) {
   // 32-bit buffer offsets into a block's output rows.
   if ((2 * kScaledTokens + 1LL) * a.out_stride * 4 + 4LL * a.rows >= 0x7FFFFFF0LL) return launch_gemm(stream, a);
-  const int wave_tiles = scaled_row_tiles(a.m, a.rows, a.n);
+  const int wave_tiles = gemm_scaled_row_tiles(a.m, a.rows, a.n);
   if (wave_tiles == 0) return launch_gemm(stream, a);
   const ScaledWork w = scaled_work(a.m, a.rows, a.n);
   unsigned char* base = static_cast<unsigned char*>(work);

@@ -141,6 +141,7 @@ hipError_t launch_gemm_wide(hipStream_t stream, const GemmArgs& a);
 // Long-prompt token GEMM on the block-scaled FP6 x FP4 MFMA: the same order.
 // Bytes of workspace it needs (16-byte aligned), 0 where it does not apply.
 size_t gemm_scaled_work(int m, int rows, int n);
+int gemm_scaled_row_tiles(int m, int rows, int n);  // 32-row tiles per wave (1..3), 0 = does not apply
 hipError_t launch_gemm_scaled(hipStream_t stream, const GemmArgs& a, void* work);
 // Long-prompt token GEMM split four ways along K (few output rows); its fp32
 // order is four contiguous group ranges added in order.

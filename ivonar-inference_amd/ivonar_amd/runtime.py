@@ -112,6 +112,8 @@ def library() -> ctypes.CDLL:
             lib.ivonar_stream_read_sink_words.restype = c_int
             lib.ivonar_gemm_work.argtypes = [c_int, c_int, c_int]
             lib.ivonar_gemm_work.restype = c_longlong
+            lib.ivonar_gemm_row_tiles.argtypes = [c_int, c_int, c_int]
+            lib.ivonar_gemm_row_tiles.restype = c_int
             lib.ivonar_linear_work.argtypes = [c_int, c_int, c_int, c_int]
             lib.ivonar_linear_work.restype = c_longlong
             lib.ivonar_linear_half.argtypes = [c_int, c_void_p]
