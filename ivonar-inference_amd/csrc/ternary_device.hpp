@@ -379,6 +379,18 @@ __device__ __forceinline__ unsigned quantize4(const float (&x)[4], float inv, fl
   return biased ^ 0x80808080u;
 }
 
+// The same four bytes by the division itself.  A thread with few inputs has the
+// reciprocal's own latency and the guard's branch to pay and little to save: the
+// GEMV prologues divide where a thread holds four inputs (or, read as float4,
+// eight).  24 layers of d=1024, ffn 4096: 3068 -> 3104 tokens/s, 8 layers of
+// d=2048, ffn 8192: 6775 -> 6845 (dividing everywhere: 3104 and 6685).
+__device__ __forceinline__ unsigned quantize4_divide(const float (&x)[4], float scale) {
+  unsigned q4 = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) q4 |= ((unsigned)(int)__builtin_rintf(x[e] / scale) & 0xffu) << (8 * e);
+  return q4;
+}
+
 // The q8 words of a 16-input quad from its four lanes' bytes (lanes 4g .. 4g+3,
 // lane j holds inputs 4j .. 4j+3): word k of the quad takes byte k of lane i
 // at byte i, so lane j forms word j with three DPP quad permutations and two
@@ -564,7 +576,7 @@ __device__ __forceinline__ float quantize_row_to_lds(const RowSource& src, int c
       float e4[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) e4[e] = (4 * c + e) * kThreads + tid < n ? v[4 * c + e] : 0.0f;
-      const unsigned q4 = quantize4(e4, inv, scale);
+      const unsigned q4 = NB == 4 ? quantize4_divide(e4, scale) : quantize4(e4, inv, scale);
       const unsigned pa = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x124, 0xF, 0xF, false);
       const unsigned pb = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x128, 0xF, 0xF, false);
       const unsigned pc = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x12C, 0xF, 0xF, false);
@@ -622,7 +634,7 @@ __device__ __forceinline__ float quantize_plain_row4_to_lds(const RowSource& src
     const int f = c * kThreads + tid;
     const float e[4] = {v[c].x, v[c].y, v[c].z, v[c].w};
     // Inputs past the row (f >= n4) hold zeros, which quantize to 0.
-    const unsigned word = transpose.word(quantize4(e, inv, scale));
+    const unsigned word = transpose.word(NC <= 2 ? quantize4_divide(e, scale) : quantize4(e, inv, scale));
     if (f < chunks * 16) {  // whole quads: chunks * 16 is a multiple of 4
       const int g = f >> 2;  // quad g: chunk g >> 2, quad g & 3
       reinterpret_cast<unsigned*>(lds_q)[(((g & 3) * chunks + (g >> 2)) << 2) + j] = word;
