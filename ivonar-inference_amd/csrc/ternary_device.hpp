@@ -383,7 +383,9 @@ __device__ __forceinline__ unsigned quantize4(const float (&x)[4], float inv, fl
 // reciprocal's own latency and the guard's branch to pay and little to save: the
 // GEMV prologues divide where a thread holds four inputs (or, read as float4,
 // eight).  24 layers of d=1024, ffn 4096: 3068 -> 3104 tokens/s, 8 layers of
-// d=2048, ffn 8192: 6775 -> 6845 (dividing everywhere: 3104 and 6685).
+// d=2048, ffn 8192: 6775 -> 6845 (dividing everywhere: 3104 and 6685).  Where
+// many blocks keep a CU's VALU busy the reciprocal wins at any length (2048
+// rows of 1024 in quantize_row_kernel: 5.0 us, 5.25 with the division).
 __device__ __forceinline__ unsigned quantize4_divide(const float (&x)[4], float scale) {
   unsigned q4 = 0;
 #pragma unroll
@@ -510,12 +512,13 @@ __device__ __forceinline__ int chunk_lane_sum(int v) {
 // The q8 bytes go to LDS in the quad-planar layout (quad w of chunk u at
 // 16-byte slot w*C + u; word k of a quad holds inputs 16w + k + 4b' at byte
 // b'), zero past n up to C*64.  Returns the token scale.  All threads of the
-// block call it; it ends with the block's writes not yet fenced.
+// block call it; it ends with the block's writes not yet fenced.  ROWS: in a
+// launch of its own, where many rows may share a CU (see quantize4_divide).
 struct NoLoads {
   __device__ void operator()() const {}
 };
 
-template <int MODE, int NB = kBatch, typename In = float, typename AfterLoads = NoLoads>
+template <int MODE, int NB = kBatch, typename In = float, bool ROWS = false, typename AfterLoads = NoLoads>
 __device__ __forceinline__ float quantize_row_to_lds(const RowSource& src, int chunks, unsigned char* lds_q,
                                                      float* slots, AfterLoads after_loads = AfterLoads{}) {
   static_assert(MODE == kPlain || MODE == kNorm, "register path for PLAIN and NORM rows");
@@ -576,7 +579,7 @@ __device__ __forceinline__ float quantize_row_to_lds(const RowSource& src, int c
       float e4[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) e4[e] = (4 * c + e) * kThreads + tid < n ? v[4 * c + e] : 0.0f;
-      const unsigned q4 = NB == 4 ? quantize4_divide(e4, scale) : quantize4(e4, inv, scale);
+      const unsigned q4 = NB == 4 && !ROWS ? quantize4_divide(e4, scale) : quantize4(e4, inv, scale);
       const unsigned pa = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x124, 0xF, 0xF, false);
       const unsigned pb = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x128, 0xF, 0xF, false);
       const unsigned pc = (unsigned)__builtin_amdgcn_mov_dpp((int)q4, 0x12C, 0xF, 0xF, false);

@@ -82,3 +82,20 @@ def test_attn_rows(cuda, oracle, head_dim, heads, splits):
                                             in_stride=stride))
     finally:
         runtime.library().ivonar_define(b"HEAD_DIM", 64)
+
+
+@pytest.mark.parametrize("mode", ["plain", "norm"])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 191, 255, 256, 257])
+def test_rows_of_one_input_per_thread(cuda, oracle, mode, n):
+    """Up to 256 inputs a thread holds one; 256 is the last such row."""
+    import torch
+    from ivonar_amd import ops
+
+    rng = np.random.default_rng(n)
+    x = _rows(rng, 5, n)
+    rows = torch.full((5 * (n + 1) + 1,), 7.0, device=cuda)[1:].view(5, n + 1)[:, :n]
+    rows.copy_(torch.from_numpy(x))
+    weight = (1.0 + 0.1 * rng.standard_normal(n)).astype(np.float32) if mode == "norm" else None
+    code = ops.MODE_NORM if mode == "norm" else ops.MODE_PLAIN
+    actual = ops.quantize_rows(rows, mode=code, n=n, aux=None if weight is None else torch.from_numpy(weight).to(cuda))
+    _check(actual, oracle.quantize_rows(T.MODE_NORM if mode == "norm" else T.MODE_PLAIN, x, n, aux=weight, eps=1e-6))
