@@ -4,7 +4,9 @@
 // One block owns one token row and reads it once: the row stays in registers
 // from the absmax (and the sum of squares or the split-softmax merge before
 // it) to the int8 values, so a row costs one memory round trip, whatever its
-// mode.  What bounds these kernels: for one to a dozen rows the chain of
+// mode.  Where rows are few and long, several blocks share a row's conversions
+// instead, each reading the row for its absmax (few_long_rows and
+// launch_plain_shape say from where on).  What bounds these kernels: for one to a dozen rows the chain of
 // latencies (launch, one round trip, one or two block reductions), from some
 // hundred rows on the bytes read.
 //
@@ -15,8 +17,9 @@
 //     boundary (quantize_row_kernel, up to 8192 inputs);
 //   * ATTN rows of up to 16384 inputs (quantize_attn_kernel): the softmax
 //     weight of every (head, split) is formed once, in LDS, not once per input;
-//   * anything longer: quantize_rows_kernel, one block per slice of 16 chunks,
-//     which first reduces the whole row and then quantizes its slice.
+//   * anything longer, and few long rows of the second kind: quantize_rows_kernel,
+//     one block per slice of 16 chunks, which first reduces the whole row and
+//     then quantizes its slice.
 //
 // Measured (one MI355X, time per launch in a chain of them, before with the
 // slice kernel or clamped duplicate loads -> now): 2048 x 4096 PLAIN 15.6 ->
@@ -38,9 +41,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows_kernel(QuantArgs a) {
   const int chunks = (a.n + kChunk - 1) / kChunk;
   const RowSource src{a.input + (size_t)t * a.in_stride, a.aux, a.n, a.eps, a.splits, a.head_dim};
   float inv_rms;
-  // Rows of up to 1024 inputs (the decoder's model width) load 4 inputs per
-  // thread and pass, not 16 mostly clamped ones (one block-uniform branch).
-  const float scale = a.n <= 4 * kThreads ? row_scale<MODE, 4>(src, inv_rms, slots) : row_scale<MODE>(src, inv_rms, slots);
+  const float scale = row_scale<MODE>(src, inv_rms, slots);
   const int word = threadIdx.x;
   const int u = blockIdx.x * kSliceChunks + (word >> 4);
   int value = 0;
@@ -319,8 +320,23 @@ bool launch_row(hipStream_t stream, const QuantArgs& a) {
 // either way).
 constexpr int kManyRows = 256;
 
+// Whether rows of more than `least` and up to `most` inputs go to the slice
+// kernel: so few of them that `per_cu` of its blocks per CU hold all slices.
+// A row's conversions are then shared by its slices, which saves more than
+// their repeated reads of the row cost.  PLAIN rows off a 16-byte boundary,
+// slices against one block per row: 12 x 8190 3.0 and 4.3 us, 12 x 2050 2.7 and
+// 3.2, 100 x 8190 4.1 and 4.5, 256 x 4096 3.6 both, 150 x 8190 7.7 and 4.7.  NORM
+// rows read the row three times in slices: 12 x 8190 4.5 and 5.0 us, 40 x 4096
+// 3.6 and 3.9, 64 x 4097 5.6 and 5.0; read as float4 only past 3072 inputs (12 x
+// 4096 3.5 and 3.7, 12 x 3072 3.6 both).
+bool few_long_rows(const QuantArgs& a, int least, int most, int per_cu) {
+  if (a.n <= least || a.n > most || a.m > kManyRows) return false;
+  return (long long)a.m * ceil_div(a.n, kSliceChunks * kChunk) <= (long long)per_cu * device_cus();
+}
+
 bool launch_norm(hipStream_t stream, const QuantArgs& a, bool aligned) {
   const int n4 = a.n >> 2;
+  if (aligned ? few_long_rows(a, 3072, 4096, 1) : few_long_rows(a, 8 * kThreads, 32 * kThreads, 1)) return false;
   if (!aligned || n4 <= 256 || (reinterpret_cast<uintptr_t>(a.aux) & 15) != 0) return launch_row<kNorm>(stream, a);
   const dim3 grid(1, a.m);
   const bool many = a.m >= kManyRows;
@@ -336,9 +352,14 @@ bool launch_norm(hipStream_t stream, const QuantArgs& a, bool aligned) {
 template <int T, int NC, typename In>
 void launch_plain_shape(hipStream_t stream, const QuantArgs& a) {
   // Few long rows: one CU would spend more time on a row's conversions than on
-  // its absmax (12 rows of 28672: 5.4 us with one block per row, 3.5 with eight).
-  if (NC > 1 && (long long)a.m * NC <= 2LL * device_cus())
-    hipLaunchKernelGGL((quantize_plain_kernel<T, NC, (NC > 1), In>), dim3(NC, a.m), dim3(T), 0, stream, a);
+  // its absmax (12 rows of 28672: 5.4 us with one block per row, 3.5 with its
+  // seven slices).  Slices past one block per CU cost more than they share out
+  // (40 rows of 28672: 7.3 us in slices, 5.5 in rows; 80 of 9000: 4.1, 3.3 with
+  // three slices instead of four).
+  int slices = ceil_div(ceil_div(a.n, kChunk) * 16, T);
+  if (NC == 4 && (long long)a.m * NC <= device_cus()) slices = NC;  // one of them empty or not: 2.9 us, 3.0 with three
+  if (NC > 1 && (long long)a.m * slices <= device_cus())
+    hipLaunchKernelGGL((quantize_plain_kernel<T, NC, (NC > 1), In>), dim3(slices, a.m), dim3(T), 0, stream, a);
   else
     hipLaunchKernelGGL((quantize_plain_kernel<T, NC, false, In>), dim3(1, a.m), dim3(T), 0, stream, a);
 }
@@ -401,7 +422,10 @@ hipError_t launch_quantize(hipStream_t stream, const QuantArgs& a) {
   const bool aligned = (a.n & 3) == 0 && (a.in_stride & 3) == 0 && (reinterpret_cast<uintptr_t>(a.input) & 15) == 0;
   bool launched = false;
   switch (a.mode) {
-    case kPlain: launched = aligned ? launch_plain<float>(stream, a) : launch_row<kPlain>(stream, a); break;
+    case kPlain:
+      if (aligned) launched = launch_plain<float>(stream, a);
+      else if (!few_long_rows(a, 8 * kThreads, 32 * kThreads, 4)) launched = launch_row<kPlain>(stream, a);
+      break;
     case kNorm: launched = launch_norm(stream, a, aligned); break;
     case kAttn: launched = launch_attn(stream, a); break;
     default: return hipErrorInvalidValue;

@@ -84,6 +84,35 @@ def test_attn_rows(cuda, oracle, head_dim, heads, splits):
         runtime.library().ivonar_define(b"HEAD_DIM", 64)
 
 
+# Rows on both sides of the rules that hand few long rows to several blocks: PLAIN rows of float4 in slices of 4096
+# inputs (fewer than the register layout has room for, a last one in part), rows off a 16-byte boundary and NORM
+# rows in the slice kernel or in one block each.
+@pytest.mark.parametrize("m,n,offset", [(36, 28672, 0), (37, 28672, 0), (51, 20000, 0), (52, 20000, 0), (85, 9000, 0),
+                                        (86, 9000, 0), (65, 12292, 0), (128, 8192, 0), (129, 8192, 0), (257, 2050, 0),
+                                        (256, 4096, 1), (257, 4096, 1), (204, 4097, 0), (205, 4097, 0), (129, 8191, 0)])
+def test_plain_rows_shared_by_blocks(cuda, oracle, m, n, offset):
+    import torch
+    from ivonar_amd import ops
+
+    x = _rows(np.random.default_rng(m + n), m, n)
+    rows = torch.empty(m * n + offset, device=cuda)[offset:].view(m, n)
+    rows.copy_(torch.from_numpy(x))
+    _check(ops.quantize_rows(rows), oracle.quantize_rows(T.MODE_PLAIN, x, n))
+
+
+@pytest.mark.parametrize("m,n", [(64, 4096), (65, 4096), (64, 3076), (3, 3072), (51, 4097), (52, 4097), (32, 8191),
+                                 (33, 8191), (86, 2051)])
+def test_norm_rows_shared_by_blocks(cuda, oracle, m, n):
+    import torch
+    from ivonar_amd import ops
+
+    rng = np.random.default_rng(m + n)
+    x = _rows(rng, m, n)
+    weight = (1.0 + 0.1 * rng.standard_normal(n)).astype(np.float32)
+    actual = ops.quantize_rows(torch.from_numpy(x).to(cuda), mode=ops.MODE_NORM, aux=torch.from_numpy(weight).to(cuda))
+    _check(actual, oracle.quantize_rows(T.MODE_NORM, x, n, aux=weight, eps=1e-6))
+
+
 @pytest.mark.parametrize("mode", ["plain", "norm"])
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 191, 255, 256, 257])
 def test_rows_of_one_input_per_thread(cuda, oracle, mode, n):
