@@ -325,7 +325,9 @@ constexpr int kManyRows = 256;
 // A row's conversions are then shared by its slices, which saves more than
 // their repeated reads of the row cost.  PLAIN rows off a 16-byte boundary,
 // slices against one block per row: 12 x 8190 3.0 and 4.3 us, 12 x 2050 2.7 and
-// 3.2, 100 x 8190 4.1 and 4.5, 256 x 4096 3.6 both, 150 x 8190 7.7 and 4.7.  NORM
+// 3.2, 60 x 8190 3.5 and 4.4, 150 x 8190 7.7 and 4.7; between two and four blocks
+// per CU slices still finish first (100 x 8190 4.1 and 4.5) but the GEMM behind
+// them then takes longer than they save (77 x 8190 -> 4100: 22.5 and 20.6).  NORM
 // rows read the row three times in slices: 12 x 8190 4.5 and 5.0 us, 40 x 4096
 // 3.6 and 3.9, 64 x 4097 5.6 and 5.0; read as float4 only past 3072 inputs (12 x
 // 4096 3.5 and 3.7, 12 x 3072 3.6 both).
@@ -424,7 +426,7 @@ hipError_t launch_quantize(hipStream_t stream, const QuantArgs& a) {
   switch (a.mode) {
     case kPlain:
       if (aligned) launched = launch_plain<float>(stream, a);
-      else if (!few_long_rows(a, 8 * kThreads, 32 * kThreads, 4)) launched = launch_row<kPlain>(stream, a);
+      else if (!few_long_rows(a, 8 * kThreads, 32 * kThreads, 2)) launched = launch_row<kPlain>(stream, a);
       break;
     case kNorm: launched = launch_norm(stream, a, aligned); break;
     case kAttn: launched = launch_attn(stream, a); break;

@@ -88,8 +88,9 @@ def test_attn_rows(cuda, oracle, head_dim, heads, splits):
 # inputs (fewer than the register layout has room for, a last one in part), rows off a 16-byte boundary and NORM
 # rows in the slice kernel or in one block each.
 @pytest.mark.parametrize("m,n,offset", [(36, 28672, 0), (37, 28672, 0), (51, 20000, 0), (52, 20000, 0), (85, 9000, 0),
-                                        (86, 9000, 0), (65, 12292, 0), (128, 8192, 0), (129, 8192, 0), (257, 2050, 0),
-                                        (256, 4096, 1), (257, 4096, 1), (204, 4097, 0), (205, 4097, 0), (129, 8191, 0)])
+                                        (86, 9000, 0), (65, 12292, 0), (128, 8192, 0), (129, 8192, 0), (170, 2050, 0),
+                                        (171, 2050, 0), (128, 4096, 1), (129, 4096, 1), (102, 4097, 0), (103, 4097, 0),
+                                        (64, 8191, 0), (65, 8191, 0)])
 def test_plain_rows_shared_by_blocks(cuda, oracle, m, n, offset):
     import torch
     from ivonar_amd import ops
