@@ -34,6 +34,26 @@ def test_half_rows(cuda, dtype, m, k):
     assert ops.ternary_linear(batched, matrix).shape == (1, m, 130)
 
 
+@pytest.mark.parametrize("m,k", [(64, 1101), (65, 1101), (65, 8190), (65, 1100), (2, 8194), (70, 8194)])
+def test_strided_rows(cuda, m, k):
+    """One copy at most before the call (the half types are converted by it or by the quantizer): the bits of the
+    rows converted first, for each type."""
+    import torch
+    from ivonar_amd import ops
+
+    rng = np.random.default_rng(m + k)
+    _, packed, scale_bits, _ = make_layer(rng, 130, k)
+    matrix = device_matrix(packed, scale_bits, k, device=cuda)
+    wide = torch.randn(m, k + 6, device=cuda)
+    for dtype in (torch.float16, torch.bfloat16, torch.float64, torch.float32):
+        x = wide.to(dtype)[:, 3:3 + k]
+        expected = ops.ternary_linear(x.float().contiguous(), matrix)
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as trace:
+            y = ops.ternary_linear(x, matrix)
+        assert torch.equal(y, expected), dtype
+        assert sum(event.count for event in trace.key_averages() if event.key == "aten::copy_") == 1, dtype
+
+
 def test_linear_matches_the_separate_calls(cuda):
     import torch
     from ivonar_amd import ops
