@@ -3,8 +3,7 @@
 Only the tests and ``bench.py``'s token check use this module, and only as the
 checker of the decoder's tokens and logits.
 
-It restates the decode step and the 32-token prefill tile of the decoder
-(the reference's ``kernel_decoder.py:233-269`` and ``:303-368``, without the
+It restates the decode step and the prefill tile of the decoder (the reference's ``kernel_decoder.py:233-269`` and ``:303-368``, without the
 mixers: the output projection reads the V third of the fused entry
 projection) from the oracle's primitives:
 
@@ -17,19 +16,19 @@ projection) from the oracle's primitives:
   GEMM plan), both pinned against ``orc_gemv_pairs`` / ``orc_gemm_split``.
 
 The plans are passed in as callables, ``gemv_lanes(rows, k)`` and
-``gemm_splits(m, rows, k)``; they are parameters of the kernels' summation
-order, not computations of the checker.
+``gemm_splits(m, rows, k)``, and so are the token counts a tile may have
+(``tiles``; a prompt runs in tiles of the longest and one of the smallest that
+holds the rest): they are parameters of the kernels' summation order, not
+computations of the checker.
 """
 
 from __future__ import annotations
 
-from collections.abc import Callable
+from collections.abc import Callable, Sequence
 
 import numpy as np
 
 import ternary_oracle as T
-
-TILE = 32
 
 
 class _Projection:
@@ -50,8 +49,9 @@ def _values(layer, codes) -> np.ndarray:
 
 class StackOracle:
     def __init__(self, weights, gemv_lanes: Callable[[int, int], int], gemm_splits: Callable[[int, int, int], int],
-                 oracle: T.Oracle | None = None) -> None:
+                 oracle: T.Oracle | None = None, tiles: Sequence[int] = (32,)) -> None:
         self.oracle = oracle or T.oracle()
+        self.tiles = tuple(tiles)
         self.config = weights.config
         codes = weights.codes or {}
         self._gemv_lanes = gemv_lanes
@@ -83,20 +83,21 @@ class StackOracle:
     # ----------------------------------------------------------------- one linear
 
     def _linear(self, projection: _Projection, x: np.ndarray, mode: int, aux, epi: int, out: np.ndarray,
-                tile: bool) -> np.ndarray:
-        """One projection for one token row: quantize, exact partials, fp32 finish in the kernel's order."""
+                tile: int) -> np.ndarray:
+        """One projection for one token row: quantize, exact partials, fp32 finish in the kernel's order
+        (`tile`: the tokens of the row's prefill tile, 0 in a decode step)."""
         k = projection.k
         q8, _, scale = self.oracle.quantize_rows(mode, x, k, aux=aux, eps=self.config.eps)
         partials = self.oracle.partials_i8(projection.values, T.q8_linear(q8[0], k))
         if tile:
-            splits = self._gemm_splits(TILE, projection.rows, k)  # 0: one token, run as the decode GEMV
+            splits = self._gemm_splits(tile, projection.rows, k)  # 0: one token, run as the decode GEMV
             order, param = (1, splits) if splits else (0, self._gemv_lanes(projection.rows, k))
         else:
             order, param = 0, self._gemv_lanes(projection.rows, k)
         return self.oracle.finish(order, param, epi, partials, projection.scale_bits, scale, None, out, k,
                                   out.shape[-1])
 
-    def _layer(self, ops: dict, residual: np.ndarray, tile: bool) -> None:
+    def _layer(self, ops: dict, residual: np.ndarray, tile: int) -> None:
         hidden, dense = self.config.hidden, self.config.dense
         mixer_in = np.zeros(3 * hidden, dtype=np.float32)
         self._linear(ops["qkv"], residual, T.MODE_NORM, ops["mixer_norm"], T.EPI_STORE, mixer_in, tile)
@@ -107,7 +108,7 @@ class StackOracle:
 
     def _head(self, residual: np.ndarray) -> np.ndarray:
         logits = np.zeros(self.config.vocab, dtype=np.float32)
-        return self._linear(self.token, residual, T.MODE_NORM, self.final_norm, T.EPI_STORE, logits, False)
+        return self._linear(self.token, residual, T.MODE_NORM, self.final_norm, T.EPI_STORE, logits, 0)
 
     def _embed(self, token: int) -> np.ndarray:
         return self.oracle.embed(np.array([token], dtype=np.int64), self.token_packed, self.token.scale_bits,
@@ -115,17 +116,26 @@ class StackOracle:
 
     # ----------------------------------------------------------------- decoding
 
-    def prefill_logits(self, prompt) -> np.ndarray:
-        """Logits of the prompt's last token through the tile path (rows of a tile are independent)."""
-        residual = self._embed(int(prompt[-1]))
+    def last_tile(self, length: int) -> int:
+        """Tokens of the tile that holds the last of `length` tokens."""
+        rest = (length - 1) % self.tiles[-1] + 1
+        return next(size for size in self.tiles if size >= rest)
+
+    def tile_residual(self, token: int, tile: int) -> np.ndarray:
+        """The residual a token's row of a `tile`-token tile ends with (rows of a tile are independent)."""
+        residual = self._embed(int(token))
         for ops in self.layers:
-            self._layer(ops, residual, tile=True)
-        return self._head(residual)
+            self._layer(ops, residual, tile)
+        return residual
+
+    def prefill_logits(self, prompt) -> np.ndarray:
+        """Logits of the prompt's last token through the tile path."""
+        return self._head(self.tile_residual(int(prompt[-1]), self.last_tile(len(prompt))))
 
     def step_logits(self, token: int) -> np.ndarray:
         residual = self._embed(int(token))
         for ops in self.layers:
-            self._layer(ops, residual, tile=False)
+            self._layer(ops, residual, 0)
         return self._head(residual)
 
     def generate(self, prompt, count: int, keep_logits: bool = False):

@@ -18,9 +18,10 @@ CONFIGS = {
 
 def _oracle(weights):
     from ivonar_amd import runtime
+    from ivonar_amd.decoder import TILES
     from stack_oracle import StackOracle
 
-    return StackOracle(weights, lambda rows, k: runtime.gemv_plan(rows, k)[0], runtime.gemm_plan)
+    return StackOracle(weights, lambda rows, k: runtime.gemv_plan(rows, k)[0], runtime.gemm_plan, tiles=TILES)
 
 
 @pytest.fixture(scope="module", params=sorted(CONFIGS))
@@ -123,9 +124,9 @@ def test_sampled_tokens_match_the_oracle(cuda, name):
 
 
 def test_prefill_tile_graph_matches_the_oracle(pair):
-    """After capture() every 32-token tile of a prefill is one replay of the captured tile program: the
-    logits stay bit-exact for prompts of 40, 1 and 32 tokens (two replays, then one, with eager decode steps
-    between), and greedy steps after a graph prefill give the oracle's tokens."""
+    """After capture() every tile of a prefill is one replay of the captured program of its size: the logits
+    stay bit-exact for prompts of 40, 1 and 32 tokens (a 64-token tile, then 32-token ones, with eager decode
+    steps between), and greedy steps after a graph prefill give the oracle's tokens."""
     decoder, oracle = pair
     decoder.prefill(prompt_ids(decoder.config.vocab, 8, seed=9))
     decoder.capture()

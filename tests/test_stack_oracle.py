@@ -83,3 +83,11 @@ def test_generate_is_greedy(stack):
     tokens, logits = oracle.generate(prompt, 4, keep_logits=True)
     assert tokens == [int(np.argmax(row)) for row in logits]
     np.testing.assert_array_equal(logits[1], oracle.step_logits(tokens[0]))
+
+
+@pytest.mark.parametrize("length,tile", [(1, 32), (32, 32), (33, 64), (129, 256), (1024, 1024), (1025, 32),
+                                         (1100, 128), (2048, 1024)])
+def test_last_tile(stack, length, tile):
+    weights, _ = stack
+    oracle = StackOracle(weights, _lanes, _splits, tiles=(32, 64, 128, 256, 512, 1024))
+    assert oracle.last_tile(length) == tile
