@@ -25,7 +25,8 @@ the head and the first token's selection run once, after the last tile (the
 reference runs its head in every tile and samples after the prompt).  The
 reference's tile has 32 tokens; here a tile is the smallest of ``TILES`` that
 holds what is left of the prompt, since a tile's 194 dependent launches (24
-layers) cost the same 3 to 4 us each at 32 tokens as at 256.
+layers) cost little more at many tokens than at few (3.4 us each at 32, 4.4 at
+128, 5.9 at 256, 11 at 1024).
 
 The mixers (recurrent scan, latent attention) are not part of this path: the
 output projection reads the V third of the entry projection's output instead
@@ -52,9 +53,12 @@ from .synthetic import LinearStackWeights
 
 TILE = 32
 # Tokens per prefill tile, each a launch list of its own (and a graph, after capture()).  Up to 1024 tokens
-# a tile costs less than two of half its size, padding included (24 layers of 1024/4096, graph replays of 32,
-# 64, .. 1024 tokens: 657, 722, 849, 1136, 1457, 2178 us; sizes between them, 192, 384 and 768, saved under 5%).
-# A prompt of 500 tokens took 11.25 ms in 16 tiles of 32 and takes 1.54 ms in one of 512.
+# a tile costs less than two of half its size, padding included, at every width measured (graph replays of 32,
+# 64, .. 1024 tokens, us: 24 layers of 1024/4096 657, 722, 849, 1136, 1457, 2178; 3 of 2048/8192 148, 184, 197, 247,
+# 344, 502; 2 of 4096/11008 157, 216, 239, 318, 473, 718; one of 8192/28672 280, 297, 289, 445, 764, 1210).  A prompt
+# a little past a size pays for the next one: 513 tokens in 512 + 32 would save 3% at 1024/4096 and 14% at
+# 8192/28672.  Sizes in between, 192, 384 and 768, saved under 5% at 1024/4096.  500 tokens of 24 layers of
+# 1024/4096 took 11.25 ms in 16 tiles of 32 and take 1.5 ms in one of 512.
 TILES = (32, 64, 128, 256, 512, 1024)
 SELF_CHECK_TOLERANCE = 0.25  # kernel_decoder.py:38
 THREADS = 256
@@ -130,8 +134,8 @@ class StackDecoder:
         self.sampler = DeviceSampler(vocab, device, max_top_k) if sampling else None
         self.uniforms = torch.zeros(self.burst, **f32)
         self.drawn_uniforms: list[float] = []  # with sampling: the uniform of every token advance_many returned
-        # prefill tile buffers (kernel_decoder.py:308-319), for the longest tile: the count of valid tokens and
-        # their ids in one buffer, filled by one copy per tile
+        # prefill tile buffers (kernel_decoder.py:308-319), for the longest tile (38 MB at 1024/4096, 283 MB at
+        # 8192/28672): the count of valid tokens and their ids in one buffer, filled by one copy per tile
         longest = TILES[-1]
         self._tile_host = torch.zeros(1 + longest, dtype=torch.int64)
         self.tile_input = torch.zeros(1 + longest, dtype=torch.int64, device=device)
@@ -399,8 +403,8 @@ class StackDecoder:
         """Runs one prompt through the prefill tiles and through single decode steps and requires both to
         agree (kernel_decoder.py:524-549), so a GPU the kernels do not run correctly on fails while loading.
 
-        The prompt has TILE + TILE // 2 + 1 random ids in [2, vocab): prefill() takes it whole (the tile
-        GEMMs), then the first id alone, after which every further id is written into the ring slot the
+        The prompt has TILE + TILE // 2 + 1 random ids in [2, vocab): prefill() takes it whole (the GEMMs of
+        a 64-token tile), then the first id alone, after which every further id is written into the ring slot the
         next step reads and one step consumes it (the GEMVs).  Both end with the logits of the prompt's last
         id; they must be finite, not all zero, and within a relative norm of SELF_CHECK_TOLERANCE, and the
         token the last step selected must lie in the vocabulary.  The decoder is reset afterwards.  Raises
