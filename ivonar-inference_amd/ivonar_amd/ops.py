@@ -63,17 +63,6 @@ def _call(name: str, device: torch.device, *args) -> None:
         check(status, name)
 
 
-def _workspace(size: int, least: int, device: torch.device) -> tuple[Tensor | None, int]:
-    """A workspace of `size` bytes, or of `least` where the device has not that much left: the entry points then
-    run the kernels that need no more, so a call never fails for the workspace of a faster kernel."""
-    if size > least:
-        try:
-            return torch.empty(size, dtype=torch.uint8, device=device), size
-        except torch.OutOfMemoryError:
-            pass
-    return (torch.empty(least, dtype=torch.uint8, device=device) if least else None), least
-
-
 def activation_buffers(m: int, n: int, device: torch.device) -> tuple[Tensor, Tensor, Tensor]:
     chunks = (n + CHUNK - 1) // CHUNK
     return (
@@ -155,7 +144,12 @@ def gemm(
     stride = int(out_stride if out_stride is not None else (out.stride(0) if out.ndim == 2 else width))
     code = _GEMM_EPILOGUES[epilogue]
     need = library().ivonar_gemm_work(rows, matrix.rows, matrix.in_features) if rows >= 128 else 0
-    work, need = _workspace(need, 0, device)
+    work = None
+    if need:
+        try:
+            work = torch.empty(need, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            need = 0  # the int8 kernels need none
     _call("ivonar_gemm", device, code, q8.data_ptr(), xsum.data_ptr(), scale.data_ptr(), matrix.packed.data_ptr(),
           matrix.scales.data_ptr(), _address(matrix.bias), out.data_ptr(), matrix.rows, matrix.in_features,
           matrix.row_bytes, matrix.groups, stride, rows, _address(work), need)
@@ -229,7 +223,13 @@ def ternary_linear(x: Tensor, matrix: Matrix) -> Tensor:
     out = torch.empty((*lead, matrix.rows), dtype=torch.float32, device=device)
     # q8 rows, chunk sums and token scales of the call, and what its GEMM needs
     need = library().ivonar_linear_work(dtype, m, matrix.rows, width)
-    work, need = _workspace(need, min(need, (m * (matrix.chunks * (CHUNK + 4) + 4) + 15) & ~15), device)
+    work = None
+    if need:
+        try:
+            work = torch.empty(need, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:  # the rows alone: the int8 kernels need no more
+            need = (m * (matrix.chunks * (CHUNK + 4) + 4) + 15) & ~15
+            work = torch.empty(need, dtype=torch.uint8, device=device)
     _call("ivonar_linear", device, rows.data_ptr(), dtype, m, _address(work), need, matrix.packed.data_ptr(),
           matrix.scales.data_ptr(), _address(matrix.bias), out.data_ptr(), matrix.rows, width, matrix.row_bytes,
           matrix.groups)
