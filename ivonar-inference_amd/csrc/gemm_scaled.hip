@@ -543,14 +543,20 @@ int gemm_scaled_row_tiles(int m, int rows, int n) {
   constexpr StepTimes kStep[3] = {
       {0.124f, 0.277f, 0.396f, 0.586f}, {0.416f, 0.599f, 0.769f, 1.05f}, {0.568f, 0.889f, 1.2f, 1.51f}};
   int choice = 0;
+  float times[4];
   for (int tiles = 1; tiles <= 3; ++tiles) {
     const long long blocks = (long long)ceil_div(rows, block_rows(tiles)) * ceil_div(m, kScaledTokens);
-    const float time = (float)padded_groups(groups) * round_time(blocks, cus, kStep[tiles - 1]) + lay_out;
-    if (time < best) {
-      best = time;
+    times[tiles] = (float)padded_groups(groups) * round_time(blocks, cus, kStep[tiles - 1]) + lay_out;
+    if (times[tiles] < best) {
+      best = times[tiles];
       choice = tiles;
     }
   }
+  // Over more than one round of blocks three tiles gain on two when the call is not repeated on the same
+  // buffers (two inputs and weights in turn, quantizer included, us, two and three tiles: 4096 -> 14336 at 4096
+  // tokens 278 and 273, 4096 -> 22016 at 2048 223 and 218, 8192 -> 28672 at 2048 520 and 501).
+  const long long pairs = (long long)ceil_div(rows, block_rows(2)) * ceil_div(m, kScaledTokens);
+  if (choice == 2 && pairs > 2LL * cus && times[3] <= 1.03f * times[2]) choice = 3;
   return choice;
 }
 
