@@ -40,11 +40,13 @@
 // Measured (one MI355X, graph replays, the lay-out's 10 us included, the int8
 // kernel before): K=4096 -> N=14336 at M=2048 168 -> 137 us (1.75 POPS); K=4096
 // -> N=22016 at M=777 123 -> 93; K=11008 -> N=4096 at M=777 72 -> 55.
-// What bounds it: the SIMD's issue port.  An MFMA holds it for about 20 of its
-// 32 cycles and each of the 5.5 VALU instructions per MFMA (4 of fold, 1.5 of
-// expansion) for 4; without its loads the kernel still takes 92% of the time,
-// without the copies of operands and per-group addresses that an earlier form
-// had it gained 8%.
+// What bounds it (counters at K=4096 -> N=14336, M=2048): one MFMA per 69 cycles
+// and SIMD over the dispatch, of which it takes 32; an instruction is in issue in
+// 68% of the cycles (MFMA and VALU 48%; 6.4 VALU per MFMA, 4 of them the fold,
+// 1.5 the expansion), and the two waves of a SIMD, which meet at a barrier per
+// group, wait for LDS, memory or it in 19% of theirs.  No bank conflicts.
+// Without its loads the kernel still takes 92% of the time; without the copies
+// of operands and the per-group addresses of an earlier form it gained 8%.
 #include <type_traits>
 
 #include "buffer_ops.hpp"
