@@ -1,7 +1,7 @@
 """Greedy decoding of a ternary linear stack on the CPU.  TEST INFRASTRUCTURE ONLY.
 
 Only the tests and ``bench.py``'s token check use this module, and only as the
-checker of the decoder's tokens and logits.
+reference of the decoder's tokens and logits.
 
 It restates the decode step and the prefill tile of the decoder (the reference's ``kernel_decoder.py:233-269`` and ``:303-368``, without the
 mixers: the output projection reads the V third of the fused entry
@@ -19,7 +19,7 @@ The plans are passed in as callables, ``gemv_lanes(rows, k)`` and
 ``gemm_splits(m, rows, k)``, and so are the token counts a tile may have
 (``tiles``; a prompt runs in tiles of the longest and one of the smallest that
 holds the rest): they are parameters of the kernels' summation order, not
-computations of the checker.
+computations of the oracle.
 """
 
 from __future__ import annotations
