@@ -3,7 +3,8 @@
 Only the tests and ``bench.py``'s token check use this module, and only as the
 reference of the decoder's tokens and logits.
 
-It restates the decode step and the prefill tile of the decoder (the reference's ``kernel_decoder.py:233-269`` and ``:303-368``, without the
+It restates the decode step and the prefill tile of the decoder (the
+reference's ``kernel_decoder.py:233-269`` and ``:303-368``, without the
 mixers: the output projection reads the V third of the fused entry
 projection) from the oracle's primitives:
 
